@@ -272,6 +272,25 @@ int mq_attn_pad_correct(const void *o, int64_t batch, int heads, int64_t rows, i
                         int64_t lse_head_stride, const float *npad, void *out, int64_t out_batch_stride, int64_t ldo,
                         float *guard, void *stream);
 
+/* Joint attention of a DiT block: for each of `batch` elements and `heads`
+ * heads of head_dim 128, softmax(q k^T / sqrt(128)) v over bf16 q, k, v
+ * (contiguous [batch, heads, l_total, 128]), rows and keys 0 .. valid - 1
+ * (later rows are padding), with f32 scores, softmax and sums.  drop (host
+ * memory, read during the call), if not NULL, holds [lo, hi) per element: the
+ * keys masked out of it (a shorter prompt's padding).  out bf16, row r and
+ * head h of element b at b * out_batch_stride + r * ldo + h * 128.  lse (f32
+ * [batch, heads, valid], or NULL) receives the log-sum-exp over the kept keys
+ * and the l_total - valid + hi - lo padded and masked ones counted as zero
+ * scores; *guard (f32 >= 0, or NULL) is raised to the largest share of a
+ * row's mass those zero scores would hold (what mq_attn_pad_correct reports).
+ * Buffers 16-byte aligned, out's strides multiples of 8 elements.  Replaces
+ * attention() at crates/mold-inference/src/flux/offload.rs:39-54 and
+ * crates/mold-inference/src/qwen_image/quantized_transformer.rs:804-823.
+ * Asynchronous on stream. */
+int mq_attention_bf16(const void *q, const void *k, const void *v, int64_t batch, int heads, int64_t l_total,
+                      int head_dim, int64_t valid, const int64_t *drop, void *out, int64_t out_batch_stride,
+                      int64_t ldo, float *lse, float *guard, void *stream);
+
 /* Quantize activations once for several Q4_K GEMVs: x [m, k] (F32 or BF16,
  * row stride ldx, 16-byte aligned rows) -> m * k / 256 blocks of
  * MQ_X_Q8K_BLOCK_BYTES at dst (16-byte aligned), by the Q8_K quantization

@@ -30,7 +30,7 @@ each gated residual update x + gate * linear(h) is the GEMM's epilogue
 (Linear.gated_add, updating x in place); a tensor whose only consumer is a quantized GEMM is produced directly in bf16
 (the GEMM rounds its input to bf16 with round-to-nearest-even either way, so
 the f32 -> bf16 staging pass disappears); attention runs in bf16 with f32
-softmax accumulation (PyTorch's fused attention) rather than as three f32 ops;
+softmax accumulation (mq_attention_bf16) rather than as three f32 ops;
 and every block's adaLN modulation linear, which reads the same silu(vec),
 runs in one GEMV over the stacked modulation weights (StackedLinear) at the
 start of the forward, with outputs identical to the per-block linears.
@@ -340,25 +340,29 @@ def _no_fused_kernel(err: RuntimeError) -> bool:
                                   "invalid device function", "not compiled"))
 
 
+def _drop_ok(drop, valid: int) -> bool:
+    """A masked key range inside the valid keys that leaves one of them."""
+    return drop is None or (0 <= drop[0] <= drop[1] <= valid and drop[1] - drop[0] < valid)
+
+
 def attention_bf16(q, k, v, valid: Optional[int] = None, guard=None, drop: Optional[Tuple[int, int]] = None,
                    out=None):
     """softmax(q k^T / sqrt(d)) v for q, k, v [H, L, D] -> [valid, H*D] bf16.
 
-    Runs PyTorch's fused attention in bf16 (f32 softmax accumulation inside; on
-    ROCm that is AOTriton's `attn_fwd` kernel).  `valid` < L marks rows
-    valid .. L-1 as padding whose k and v rows are zero: the fused kernels run
-    much faster at lengths that are multiples of 256 (1.0 vs 2.0 ms at
-    24 x 7168 vs 7145 tokens on an MI355X).  Each of the n_pad zero keys adds
-    exp(0) = 1 to a row's softmax denominator Z and nothing to its numerator, so
-    with the log-sum-exp the kernel returns, out = out_pad / s with
-    s = 1 - n_pad exp(-lse), the row's share of mass on its valid keys.  That
-    division only rescales the bf16 out_pad; its error is that of s, which stays
-    far below bf16 precision while s >= PAD_MIN_SHARE.  Rows under that share
-    (every valid score below about -10) are recomputed exactly over the valid
-    keys: with `guard` None this call finds them (one host synchronization) and
-    recomputes their heads; with `guard`, a 0-dim f32 device tensor, it only
-    raises guard to the largest 1 - s seen, and the caller checks it once
-    (FluxStep.forward reruns the step unpadded if any row fell under the share).
+    Runs libmoldq's attention kernel (mq_attention_bf16: bf16 matrix products, f32
+    scores, softmax and sums) for heads of 128 on the GPU; calls it does not take
+    (fused.takes_attention: other head sizes, inputs that autograd or a transform
+    records) go to PyTorch's fused attention.  `valid` < L marks rows valid .. L-1
+    as padding whose k and v rows are zero; the kernel never reads them as keys.
+    PyTorch's kernels do: each of the n_pad zero keys adds exp(0) = 1 to a row's
+    softmax denominator, so out = out_pad / s with s = 1 - n_pad exp(-lse), the
+    row's share of mass on its valid keys, which loses precision once s falls
+    under PAD_MIN_SHARE (every valid score below about -10).  On either path such
+    rows are reported or recomputed in f32 over the valid keys: with `guard` None
+    this call finds them (one host synchronization) and recomputes their heads;
+    with `guard`, a 0-dim f32 device tensor, it only raises guard to the largest
+    1 - s seen, and the caller checks it once (FluxStep.forward reruns the step
+    unpadded if any row fell under the share).
 
     `drop` = (lo, hi) masks keys lo .. hi-1 (a text attention mask, e.g. the
     padded tail of a shorter prompt in a CFG batch): their k and v rows must be
@@ -373,12 +377,26 @@ def attention_bf16(q, k, v, valid: Optional[int] = None, guard=None, drop: Optio
     head-chunked path on the valid rows (any other error propagates).  The
     backend used is recorded in ATTENTION_BACKEND."""
     import torch
+    from .fused import attention, takes_attention
     h, l, d = q.shape
     valid = l if valid is None else valid
     qb, kb, vb = (t.to(torch.bfloat16).contiguous() for t in (q, k, v))
     n_drop = 0 if drop is None else max(0, drop[1] - drop[0])
     if out is not None and (out.shape != (valid, h * d) or out.dtype != torch.bfloat16 or out.stride(1) != 1):
         raise ValueError(f"attention_bf16: out must be bf16 [{valid}, {h * d}] with unit column stride")
+    if ATTENTION_BACKEND["name"] in (None, "fused") and 0 < valid <= l and _drop_ok(drop, valid) \
+            and (guard is None or guard.is_cuda) and takes_attention(qb, kb, vb):
+        ATTENTION_BACKEND["name"] = "fused"
+        if guard is not None or not (valid < l or n_drop):
+            return attention(qb, kb, vb, valid, drops=[drop], out=out, guard=guard if valid < l or n_drop else None)
+        lse = torch.empty((1, h, valid), dtype=torch.float32, device=q.device)
+        res = attention(qb, kb, vb, valid, drops=[drop], out=out, lse=lse)
+        bad = ((l - valid + n_drop) * torch.exp(-lse[0]) > 1.0 - PAD_MIN_SHARE).any(dim=1)
+        if bool(bad.any()):
+            heads = bad.nonzero().flatten()
+            exact = _attention_chunked(qb[heads, :valid], kb[heads, :valid], vb[heads, :valid], drop)
+            res.view(valid, h, d)[:, heads] = exact.view(valid, heads.numel(), d)
+        return res
     if ATTENTION_BACKEND["name"] in (None, "fused"):
         try:
             if valid < l or n_drop:
@@ -460,6 +478,12 @@ def attention_bf16_batch(q, k, v, valid: int, guard, drops):
                                        for b in range(b_)])
     if guard is None or ATTENTION_BACKEND["name"] not in (None, "fused"):
         return per_element()
+    from .fused import attention, takes_attention
+    if 0 < valid <= l and all(_drop_ok(dr, valid) for dr in drops) and len(drops) == b_ and guard.is_cuda \
+            and takes_attention(q, k, v):
+        ATTENTION_BACKEND["name"] = "fused"
+        padded = valid < l or any(dr is not None and dr[1] > dr[0] for dr in drops)
+        return attention(q, k, v, valid, drops=drops, guard=guard if padded else None)
     try:
         out, lse = torch.ops.aten._scaled_dot_product_efficient_attention(q, k, v, None, True)[:2]
     except RuntimeError as err:

@@ -1,12 +1,14 @@
 """Fused block glue on the device: libmoldq's row passes between the quantized
 linears (mq_adaln_modulate, mq_gelu_tanh_bf16, mq_qk_norm_rope and
-mq_attn_pad_correct in include/moldq.h).
+mq_attn_pad_correct in include/moldq.h) and their attention (mq_attention_bf16).
 
 All run on torch's current stream and allocate only their outputs.  They need
 the HIP library (no fallback); the host-CPU path of the block graphs keeps the
 equivalent torch ops.
 """
 from __future__ import annotations
+
+import ctypes
 
 from . import _lib
 from ._lib import check
@@ -91,6 +93,50 @@ def attn_pad_correct(o, lse, npad, rows: int, guard, out):
                                           out.data_ptr(), o3.stride(0), o3.stride(1), guard.data_ptr(),
                                           _stream_ptr()))
     return out
+
+
+def takes_attention(q, k, v) -> bool:
+    """Whether `attention` computes these q, k, v: bf16 [.., H, L, 128] of one shape on one
+    GPU, contiguous and 16-byte aligned, with nothing recording the call (autograd, a
+    functorch transform, forward-mode AD, a dispatch mode, a compiler): those need
+    operations PyTorch knows."""
+    import torch
+    for t in (q, k, v):
+        if type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda or t.dtype != torch.bfloat16 \
+                or t.shape != q.shape or t.device != q.device or not t.is_contiguous() or t.data_ptr() % 16:
+            return False
+        if t.requires_grad and torch.is_grad_enabled():
+            return False
+    return (q.dim() in (3, 4) and q.shape[-1] == HEAD_DIM and 0 < q.numel() and q.shape[-2] <= 1 << 23
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0
+            and torch._C._len_torch_dispatch_stack() == 0 and not torch.compiler.is_compiling())
+
+
+def attention(q, k, v, valid: int, drops=None, out=None, lse=None, guard=None):
+    """softmax(q k^T / sqrt(128)) v over rows and keys 0 .. valid-1 of bf16 [B, H, L, 128]
+    (or [H, L, 128]), element b's keys drops[b] = (lo, hi) masked out (mq_attention_bf16).
+    Returns bf16 [B, valid, H*128] ([valid, H*128]): `out` when given (unit column stride;
+    written through a temporary if its rows are not 16-byte aligned).  lse f32 [B, H, valid]
+    and guard (0-dim f32, raised) as mq_attention_bf16 describes them."""
+    import torch
+    b_ = q.shape[0] if q.dim() == 4 else 1
+    h, l = q.shape[-3], q.shape[-2]
+    shape = (b_, valid, h * HEAD_DIM) if q.dim() == 4 else (valid, h * HEAD_DIM)
+    res = out
+    if out is None or out.data_ptr() % 16 or any(s % 8 for s in out.stride()[:-1]):
+        res = torch.empty(shape, dtype=torch.bfloat16, device=q.device)
+    drop = None
+    if drops is not None and any(d is not None for d in drops):
+        drop = (ctypes.c_int64 * (2 * b_))(*[x for d in drops for x in (d or (0, 0))])
+    with torch.cuda.device(q.device):
+        check(_lib.load().mq_attention_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), b_, h, l, HEAD_DIM, valid, drop,
+                                            res.data_ptr(), res.stride(0) if res.dim() == 3 else 0, res.stride(-2),
+                                            lse.data_ptr() if lse is not None else None,
+                                            guard.data_ptr() if guard is not None else None, _stream_ptr()))
+    if out is not None and res is not out:
+        return out.copy_(res)
+    return res
 
 
 def qk_norm_rope(qkv, heads: int, q_weight, k_weight, cos, sin, q_out, k_out, v_out, row_off: int,
