@@ -137,7 +137,7 @@ int mq_qtensor_from_device(mq_ctx *ctx, int dtype, int64_t n, int64_t k,
  * QTensor::quantize / quantize_onto (crates/mold-inference/src/flux/
  * pipeline.rs:219-229, crates/mold-inference/src/flux/lora.rs:849).
  * Runs on `stream` after work already queued there and returns when the
- * blocks are in place (through the context's upload staging buffer).
+ * blocks are in place.
  * dtype F32 / F16 / BF16 stores the values themselves (rounded to nearest
  * even when narrowing): QTensor::quantize(.., F32), which mold uses for the
  * tensors a block type cannot hold (flux/pipeline.rs:223-228). */

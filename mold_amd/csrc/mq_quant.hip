@@ -14,8 +14,8 @@
 // the same bytes is unpinned: its source is not available here, and its
 // Q2_K/Q4_K/Q5_K from_float may use make_qkx1_quants instead of
 // make_qkx2_quants.  Q4_0/Q4_1/Q5_0/Q5_1/Q8_0 have a single formula.
-// One thread quantizes one block; raw blocks go to a staging buffer that the
-// upload path then permutes into the tiled device layout.
+// A thread quantizes one 32-element block, or one sub-block of a super-block,
+// and stores its fields straight into the tiled device layout.
 #include <utility>
 
 #include "mq_kernels.h"
@@ -141,50 +141,68 @@ __device__ void q_q8_0(const float *x, uint8_t *o) {
   for (int j = 0; j < 32; ++j) o[2 + j] = (uint8_t)(int8_t)roundf(x[j] * id);
 }
 
-// ------------------------------------------------------------- k-quant helpers
+// ------------------------------------------------------------- k-quant searches
+// One thread searches one sub-block (N = 32 or 16 values, all in registers);
+// the 8 or 16 threads of a super-block are neighbouring lanes.
 
-// Scale and min search over a group of n values (ggml make_qkx2_quants).
-__device__ float qkx2(int n, int nmax, const float *x, const float *w, uint8_t *L, float *the_min, uint8_t *Laux,
-                      float rmin, float rdelta, int nstep, bool use_mad) {
+// nearest_int clamped to [0, nmax] as a float.  Exact: ggml's integer steps.
+// Otherwise for |f| < 2^22, where the magic sum's ulp is 1 and nearest_int
+// rounds to the nearest even integer: two operations for the integer form's
+// six.  (A -0 in place of 0 changes no sum: they start at +0, and a product's
+// sign of zero is lost in the square or magnitude it ends in.)
+template <bool EXACT>
+__device__ __forceinline__ float nearest_clamped(float f, int nmax) {
+  if constexpr (EXACT) {
+    return (float)mx(0, mn(nmax, nearest_int(f)));
+  } else {
+    return __builtin_amdgcn_fmed3f(__builtin_rintf(f), 0.f, (float)nmax);
+  }
+}
+
+// Scale and min search over a group of N values (ggml make_qkx2_quants); the
+// quants of the best step are nearest_clamped(best_iscale * (x - best_min)).
+// VALU-bound: 16 operations per value and step (one rounded multiply and add
+// at a time, in ggml's order).
+struct Qkx2 {
+  float scale, the_min, best_iscale, best_min;
+};
+template <int N, bool MAD>
+__device__ __forceinline__ Qkx2 qkx2(int nmax, const float (&x)[N], const float (&w)[N], float rmin, float rdelta, int nstep) {
   float vmin = x[0], vmax = x[0];
   float sum_w = w[0];
   float sum_x = sum_w * x[0];
-  for (int i = 1; i < n; ++i) {
+#pragma unroll
+  for (int i = 1; i < N; ++i) {
     if (x[i] < vmin) vmin = x[i];
     if (x[i] > vmax) vmax = x[i];
     sum_w += w[i];
     sum_x += w[i] * x[i];
   }
+  const float xmin = vmin;
   if (vmin > 0) vmin = 0;
-  if (vmax == vmin) {
-    for (int i = 0; i < n; ++i) L[i] = 0;
-    *the_min = -vmin;
-    return 0.f;
-  }
+  Qkx2 r{0.f, -vmin, 0.f, 0.f};
+  if (vmax == vmin) return r;
   float iscale = nmax / (vmax - vmin);
   float scale = 1 / iscale;
   float best = 0;
-  for (int i = 0; i < n; ++i) {
-    const int l = nearest_int(iscale * (x[i] - vmin));
-    L[i] = (uint8_t)mx(0, mn(nmax, l));
-    float diff = scale * L[i] + vmin - x[i];
-    diff = use_mad ? fabsf(diff) : diff * diff;
+  r.best_iscale = iscale;
+  r.best_min = vmin;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    float diff = scale * nearest_clamped<true>(iscale * (x[i] - vmin), nmax) + vmin - x[i];
+    diff = MAD ? fabsf(diff) : diff * diff;
     best += w[i] * diff;
   }
-  if (nstep < 1) {
-    *the_min = -vmin;
-    return scale;
-  }
-  for (int is = 0; is <= nstep; ++is) {
-    iscale = (rmin + rdelta * is + nmax) / (vmax - vmin);
+  auto step = [&]<bool EXACT>() {
+    float q[N];
     float sum_l = 0, sum_l2 = 0, sum_xl = 0;
-    for (int i = 0; i < n; ++i) {
-      int l = nearest_int(iscale * (x[i] - vmin));
-      l = mx(0, mn(nmax, l));
-      Laux[i] = (uint8_t)l;
-      sum_l += w[i] * l;
-      sum_l2 += w[i] * l * l;
-      sum_xl += w[i] * l * x[i];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      q[i] = nearest_clamped<EXACT>(iscale * (x[i] - vmin), nmax);
+      const float wl = w[i] * q[i];
+      sum_l += wl;
+      sum_l2 += wl * q[i];
+      sum_xl += wl * x[i];
     }
     const float D = sum_w * sum_l2 - sum_l * sum_l;
     if (D > 0) {
@@ -195,60 +213,67 @@ __device__ float qkx2(int n, int nmax, const float *x, const float *w, uint8_t *
         this_scale = sum_xl / sum_l2;
       }
       float mad = 0;
-      for (int i = 0; i < n; ++i) {
-        float diff = this_scale * Laux[i] + this_min - x[i];
-        diff = use_mad ? fabsf(diff) : diff * diff;
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        float diff = this_scale * q[i] + this_min - x[i];
+        diff = MAD ? fabsf(diff) : diff * diff;
         mad += w[i] * diff;
       }
       if (mad < best) {
-        for (int i = 0; i < n; ++i) L[i] = Laux[i];
+        r.best_iscale = iscale;
+        r.best_min = vmin;
         best = mad;
         scale = this_scale;
         vmin = this_min;
       }
     }
+  };
+  for (int is = 0; is <= nstep; ++is) {
+    iscale = (rmin + rdelta * is + nmax) / (vmax - vmin);
+    // iscale * (x - vmin) is monotone in x, so its ends bound it (NaN takes the exact form)
+    const bool tame = fabsf(iscale * (vmax - vmin)) < 4194304.f && fabsf(iscale * (xmin - vmin)) < 4194304.f;
+    if (__all(tame)) step.template operator()<false>();
+    else step.template operator()<true>();
   }
-  *the_min = -vmin;
-  return scale;
+  r.the_min = -vmin;
+  r.scale = scale;
+  return r;
 }
 
-// Symmetric scale search with weights x^2 (ggml make_qx_quants, rmse_type 1).
-__device__ float qx_rmse1(int n, int nmax, const float *x, int8_t *L) {
+// Symmetric scale search with weights x^2 (ggml make_qx_quants, rmse_type 1);
+// the best step's quants are nmax + clamp(nearest_int(best_iscale * x)), or
+// all 0 for a group of zeros (zero set).
+template <int N>
+__device__ __forceinline__ float qx_rmse1(int nmax, const float (&x)[N], float &best_iscale, bool &zero) {
   float vmax = 0, amax = 0;
-  for (int i = 0; i < n; ++i)
+#pragma unroll
+  for (int i = 0; i < N; ++i)
     if (fabsf(x[i]) > amax) { amax = fabsf(x[i]); vmax = x[i]; }
-  if (amax < kGroupMaxEps) {
-    for (int i = 0; i < n; ++i) L[i] = 0;
-    return 0.f;
-  }
-  float iscale = -nmax / vmax;
+  zero = amax < kGroupMaxEps;
+  best_iscale = 0.f;
+  if (zero) return 0.f;
   float sumlx = 0, suml2 = 0;
-  for (int i = 0; i < n; ++i) {
-    int l = nearest_int(iscale * x[i]);
-    l = mx(-nmax, mn(nmax - 1, l));
-    L[i] = (int8_t)(l + nmax);
-    const float w = x[i] * x[i];
-    sumlx += w * x[i] * l;
-    suml2 += w * l * l;
-  }
+  auto sums = [&](float iscale) {
+    sumlx = suml2 = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      int l = nearest_int(iscale * x[i]);
+      l = mx(-nmax, mn(nmax - 1, l));
+      const float wl = x[i] * x[i];
+      sumlx += wl * x[i] * l;
+      suml2 += wl * l * l;
+    }
+  };
+  best_iscale = -nmax / vmax;
+  sums(best_iscale);
   float scale = suml2 ? sumlx / suml2 : 0.0f;
   float best = scale * sumlx;
   for (int is = -9; is <= 9; ++is) {
     if (is == 0) continue;
-    iscale = -(nmax + 0.1f * is) / vmax;
-    sumlx = suml2 = 0;
-    for (int i = 0; i < n; ++i) {
-      int l = nearest_int(iscale * x[i]);
-      l = mx(-nmax, mn(nmax - 1, l));
-      const float w = x[i] * x[i];
-      sumlx += w * x[i] * l;
-      suml2 += w * l * l;
-    }
+    const float iscale = -(nmax + 0.1f * is) / vmax;
+    sums(iscale);
     if (suml2 > 0 && sumlx * sumlx > best * suml2) {
-      for (int i = 0; i < n; ++i) {
-        const int l = nearest_int(iscale * x[i]);
-        L[i] = (int8_t)(nmax + mx(-nmax, mn(nmax - 1, l)));
-      }
+      best_iscale = iscale;
       scale = sumlx / suml2;
       best = scale * sumlx;
     }
@@ -257,27 +282,32 @@ __device__ float qx_rmse1(int n, int nmax, const float *x, int8_t *L) {
 }
 
 // Q3_K group search (ggml make_q3_quants with do_rmse).
-__device__ float q3_group(int n, int nmax, const float *x, int8_t *L) {
+template <int N>
+__device__ __forceinline__ float q3_group(int nmax, const float (&x)[N], int (&L)[N]) {
   float vmax = 0, amax = 0;
-  for (int i = 0; i < n; ++i)
+#pragma unroll
+  for (int i = 0; i < N; ++i)
     if (fabsf(x[i]) > amax) { amax = fabsf(x[i]); vmax = x[i]; }
   if (amax < kGroupMaxEps) {
-    for (int i = 0; i < n; ++i) L[i] = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) L[i] = 0;
     return 0.f;
   }
   const float iscale = -nmax / vmax;
   float sumlx = 0, suml2 = 0;
-  for (int i = 0; i < n; ++i) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
     int l = nearest_int(iscale * x[i]);
     l = mx(-nmax, mn(nmax - 1, l));
-    L[i] = (int8_t)l;
+    L[i] = l;
     const float w = x[i] * x[i];
     sumlx += w * x[i] * l;
     suml2 += w * l * l;
   }
   for (int itry = 0; itry < 5; ++itry) {
     int changed = 0;
-    for (int i = 0; i < n; ++i) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
       const float w = x[i] * x[i];
       float slx = sumlx - w * x[i] * L[i];
       if (slx > 0) {
@@ -288,7 +318,7 @@ __device__ float q3_group(int n, int nmax, const float *x, int8_t *L) {
           slx += w * x[i] * nl;
           sl2 += w * nl * nl;
           if (sl2 > 0 && slx * slx * suml2 > sumlx * sumlx * sl2) {
-            L[i] = (int8_t)nl;
+            L[i] = nl;
             sumlx = slx;
             suml2 = sl2;
             ++changed;
@@ -298,249 +328,9 @@ __device__ float q3_group(int n, int nmax, const float *x, int8_t *L) {
     }
     if (!changed) break;
   }
-  for (int i = 0; i < n; ++i) L[i] = (int8_t)(L[i] + nmax);
+#pragma unroll
+  for (int i = 0; i < N; ++i) L[i] += nmax;
   return sumlx / suml2;
-}
-
-__device__ __forceinline__ void unpack_k4(int j, const uint8_t *q, int &sc, int &m) {
-  if (j < 4) {
-    sc = q[j] & 63;
-    m = q[j + 4] & 63;
-  } else {
-    sc = (q[j + 4] & 0xF) | ((q[j - 4] >> 6) << 4);
-    m = (q[j + 4] >> 4) | ((q[j] >> 6) << 4);
-  }
-}
-
-__device__ __forceinline__ void pack_k4(uint8_t *s, int j, uint8_t ls, uint8_t lm) {
-  if (j < 4) {
-    s[j] = ls;
-    s[j + 4] = lm;
-  } else {
-    s[j + 4] = (uint8_t)((ls & 0xF) | ((lm & 0xF) << 4));
-    s[j - 4] |= (uint8_t)((ls >> 4) << 6);
-    s[j] |= (uint8_t)((lm >> 4) << 6);
-  }
-}
-
-__device__ __forceinline__ float h2f_dev(uint16_t u) { return h2f(u); }
-
-// ------------------------------------------------------------- k-quant blocks
-// Byte offsets follow the GGUF structs (see type_info in mq_common.h).
-
-__device__ void q_q2_K(const float *x, uint8_t *o) {
-  uint8_t L[256], Laux[16];
-  float wts[16], mins[16], scales[16];
-  uint8_t *sc = o, *qs = o + 16;
-  float max_scale = 0, max_min = 0;
-  for (int j = 0; j < 16; ++j) {
-    for (int l = 0; l < 16; ++l) wts[l] = fabsf(x[16 * j + l]);
-    scales[j] = qkx2(16, 3, x + 16 * j, wts, L + 16 * j, &mins[j], Laux, -0.5f, 0.1f, 15, true);
-    if (scales[j] > max_scale) max_scale = scales[j];
-    if (mins[j] > max_min) max_min = mins[j];
-  }
-  uint16_t dh, mh;
-  if (max_scale > 0) {
-    const float iscale = 15.f / max_scale;
-    for (int j = 0; j < 16; ++j) sc[j] = (uint8_t)nearest_int(iscale * scales[j]);
-    dh = f2h(max_scale / 15.f);
-  } else {
-    for (int j = 0; j < 16; ++j) sc[j] = 0;
-    dh = f2h(0.f);
-  }
-  if (max_min > 0) {
-    const float iscale = 15.f / max_min;
-    for (int j = 0; j < 16; ++j) sc[j] |= (uint8_t)(nearest_int(iscale * mins[j]) << 4);
-    mh = f2h(max_min / 15.f);
-  } else {
-    mh = f2h(0.f);
-  }
-  put16(o + 80, dh);
-  put16(o + 82, mh);
-  for (int j = 0; j < 16; ++j) {
-    const float d = h2f_dev(dh) * (sc[j] & 0xF);
-    if (!d) continue;
-    const float dm = h2f_dev(mh) * (sc[j] >> 4);
-    for (int i = 0; i < 16; ++i) {
-      const int l = nearest_int((x[16 * j + i] + dm) / d);
-      L[16 * j + i] = (uint8_t)mx(0, mn(3, l));
-    }
-  }
-  for (int j = 0; j < 256; j += 128)
-    for (int l = 0; l < 32; ++l)
-      qs[j / 4 + l] = (uint8_t)(L[j + l] | (L[j + l + 32] << 2) | (L[j + l + 64] << 4) | (L[j + l + 96] << 6));
-}
-
-__device__ void q_q3_K(const float *x, uint8_t *o) {
-  int8_t L[256];
-  float scales[16];
-  uint8_t *hmask = o, *qs = o + 32, *sc = o + 96;
-  float max_scale = 0, amax = 0;
-  for (int j = 0; j < 16; ++j) {
-    scales[j] = q3_group(16, 4, x + 16 * j, L + 16 * j);
-    if (fabsf(scales[j]) > amax) { amax = fabsf(scales[j]); max_scale = scales[j]; }
-  }
-  for (int j = 0; j < 12; ++j) sc[j] = 0;
-  uint16_t dh;
-  if (max_scale) {
-    const float iscale = -32.f / max_scale;
-    for (int j = 0; j < 16; ++j) {
-      int8_t l = (int8_t)nearest_int(iscale * scales[j]);
-      l = (int8_t)(mx(-32, mn(31, (int)l)) + 32);
-      if (j < 8) sc[j] = l & 0xF;
-      else sc[j - 8] |= (uint8_t)((l & 0xF) << 4);
-      l >>= 4;
-      sc[j % 4 + 8] |= (uint8_t)(l << (2 * (j / 4)));
-    }
-    dh = f2h(1 / iscale);
-  } else {
-    dh = f2h(0.f);
-  }
-  put16(o + 108, dh);
-  for (int j = 0; j < 16; ++j) {
-    int8_t s = j < 8 ? (int8_t)(sc[j] & 0xF) : (int8_t)(sc[j - 8] >> 4);
-    s = (int8_t)((s | (((sc[8 + j % 4] >> (2 * (j / 4))) & 3) << 4)) - 32);
-    const float d = h2f_dev(dh) * s;
-    if (!d) continue;
-    for (int i = 0; i < 16; ++i) {
-      int l = nearest_int(x[16 * j + i] / d);
-      l = mx(-4, mn(3, l));
-      L[16 * j + i] = (int8_t)(l + 4);
-    }
-  }
-  for (int j = 0; j < 32; ++j) hmask[j] = 0;
-  int m = 0;
-  uint8_t hm = 1;
-  for (int j = 0; j < 256; ++j) {
-    if (L[j] > 3) {
-      hmask[m] |= hm;
-      L[j] -= 4;
-    }
-    if (++m == 32) { m = 0; hm <<= 1; }
-  }
-  for (int j = 0; j < 256; j += 128)
-    for (int l = 0; l < 32; ++l)
-      qs[j / 4 + l] = (uint8_t)(L[j + l] | (L[j + l + 32] << 2) | (L[j + l + 64] << 4) | (L[j + l + 96] << 6));
-}
-
-template <bool FIVE>
-__device__ void q_q45_K(const float *x, uint8_t *o) {
-  constexpr int nmax = FIVE ? 31 : 15;
-  uint8_t L[256], Laux[32];
-  float wts[32], mins[8], scales[8];
-  uint8_t *sc = o + 4;
-  float max_scale = 0, max_min = 0;
-  for (int j = 0; j < 8; ++j) {
-    float sum_x2 = 0;
-    for (int l = 0; l < 32; ++l) sum_x2 += x[32 * j + l] * x[32 * j + l];
-    const float av_x = sqrtf(sum_x2 / 32);
-    for (int l = 0; l < 32; ++l) wts[l] = av_x + fabsf(x[32 * j + l]);
-    scales[j] = qkx2(32, nmax, x + 32 * j, wts, L + 32 * j, &mins[j], Laux, FIVE ? -0.5f : -1.f, 0.1f,
-                     FIVE ? 15 : 20, false);
-    if (scales[j] > max_scale) max_scale = scales[j];
-    if (mins[j] > max_min) max_min = mins[j];
-  }
-  const float inv_scale = max_scale > 0 ? 63.f / max_scale : 0.f;
-  const float inv_min = max_min > 0 ? 63.f / max_min : 0.f;
-  for (int j = 0; j < 12; ++j) sc[j] = 0;
-  for (int j = 0; j < 8; ++j) {
-    const uint8_t ls = (uint8_t)nearest_int(inv_scale * scales[j]);
-    const uint8_t lm = (uint8_t)nearest_int(inv_min * mins[j]);
-    pack_k4(sc, j, mn<uint8_t>(63, ls), mn<uint8_t>(63, lm));
-  }
-  const uint16_t dh = f2h(max_scale / 63.f), mh = f2h(max_min / 63.f);
-  put16(o, dh);
-  put16(o + 2, mh);
-  for (int j = 0; j < 8; ++j) {
-    int s, m;
-    unpack_k4(j, sc, s, m);
-    const float d = h2f_dev(dh) * s;
-    if (!d) continue;
-    const float dm = h2f_dev(mh) * m;
-    for (int i = 0; i < 32; ++i) {
-      const int l = nearest_int((x[32 * j + i] + dm) / d);
-      L[32 * j + i] = (uint8_t)mx(0, mn(nmax, l));
-    }
-  }
-  if (!FIVE) {
-    uint8_t *q = o + 16;
-    for (int j = 0; j < 256; j += 64) {
-      for (int l = 0; l < 32; ++l) q[l] = (uint8_t)(L[j + l] | (L[j + l + 32] << 4));
-      q += 32;
-    }
-  } else {
-    uint8_t *qh = o + 16, *ql = o + 48;
-    for (int j = 0; j < 32; ++j) qh[j] = 0;
-    uint8_t m1 = 1, m2 = 2;
-    for (int n = 0; n < 256; n += 64) {
-      for (int j = 0; j < 32; ++j) {
-        int l1 = L[n + j];
-        if (l1 > 15) { l1 -= 16; qh[j] |= m1; }
-        int l2 = L[n + j + 32];
-        if (l2 > 15) { l2 -= 16; qh[j] |= m2; }
-        ql[j] = (uint8_t)(l1 | (l2 << 4));
-      }
-      m1 <<= 2;
-      m2 <<= 2;
-      ql += 32;
-    }
-  }
-}
-
-__device__ void q_q6_K(const float *x, uint8_t *o) {
-  int8_t L[256];
-  float scales[16];
-  uint8_t *ql = o, *qh = o + 128;
-  int8_t *sc = reinterpret_cast<int8_t *>(o + 192);
-  float max_scale = 0, max_abs = 0;
-  for (int ib = 0; ib < 16; ++ib) {
-    scales[ib] = qx_rmse1(16, 32, x + 16 * ib, L + 16 * ib);
-    if (fabsf(scales[ib]) > max_abs) { max_abs = fabsf(scales[ib]); max_scale = scales[ib]; }
-  }
-  if (max_abs < kGroupMaxEps) {
-    for (int i = 0; i < 210; ++i) o[i] = 0;
-    put16(o + 208, f2h(0.f));
-    return;
-  }
-  const float iscale = -128.f / max_scale;
-  const uint16_t dh = f2h(1 / iscale);
-  put16(o + 208, dh);
-  for (int ib = 0; ib < 16; ++ib) sc[ib] = (int8_t)mn(127, nearest_int(iscale * scales[ib]));
-  for (int j = 0; j < 16; ++j) {
-    const float d = h2f_dev(dh) * sc[j];
-    if (!d) continue;
-    for (int i = 0; i < 16; ++i) {
-      int l = nearest_int(x[16 * j + i] / d);
-      l = mx(-32, mn(31, l));
-      L[16 * j + i] = (int8_t)(l + 32);
-    }
-  }
-  for (int j = 0; j < 256; j += 128) {
-    for (int l = 0; l < 32; ++l) {
-      const uint8_t q1 = L[j + l] & 0xF, q2 = L[j + l + 32] & 0xF;
-      const uint8_t q3 = L[j + l + 64] & 0xF, q4 = L[j + l + 96] & 0xF;
-      ql[l] = (uint8_t)(q1 | (q3 << 4));
-      ql[l + 32] = (uint8_t)(q2 | (q4 << 4));
-      qh[l] = (uint8_t)((L[j + l] >> 4) | ((L[j + l + 32] >> 4) << 2) | ((L[j + l + 64] >> 4) << 4) |
-                        ((L[j + l + 96] >> 4) << 6));
-    }
-    ql += 64;
-    qh += 32;
-  }
-}
-
-template <int TYPE>
-__device__ __forceinline__ void quant_block(const float *x, uint8_t *o) {
-  if constexpr (TYPE == Q4_0) q_q4_0(x, o);
-  else if constexpr (TYPE == Q4_1) q_q4_1(x, o);
-  else if constexpr (TYPE == Q5_0) q_q5_0(x, o);
-  else if constexpr (TYPE == Q5_1) q_q5_1(x, o);
-  else if constexpr (TYPE == Q8_0) q_q8_0(x, o);
-  else if constexpr (TYPE == Q2_K) q_q2_K(x, o);
-  else if constexpr (TYPE == Q3_K) q_q3_K(x, o);
-  else if constexpr (TYPE == Q4_K) q_q45_K<false>(x, o);
-  else if constexpr (TYPE == Q5_K) q_q45_K<true>(x, o);
-  else q_q6_K(x, o);
 }
 
 template <typename F, int... I>
@@ -562,67 +352,6 @@ __device__ __forceinline__ float e4m3_to_f32(uint8_t b) {
     return sign ? -v : v;
   }
   return __uint_as_float(sign | ((e + 120u) << 23) | (m << 20));
-}
-
-// One thread per block: copy the block's inputs to private memory (f32 as
-// given, or FP8 E4M3 decoded exactly and multiplied by `scale`; with VEC the
-// rows are 16-byte aligned and the inputs come as 16-byte loads), quantize
-// into a private block image and put it in LDS; the workgroup's 64 blocks,
-// contiguous in the raw staging buffer, then leave as 16-byte stores (one
-// byte store per output byte had left the FP8 -> Q8_0 pass at ~7 % of HBM).
-template <int TYPE, bool FP8, bool VEC>
-__global__ __launch_bounds__(64) void quantize_kernel(const void *__restrict__ src, int64_t ld, int64_t n,
-                                                      int64_t nb, float scale, uint8_t *__restrict__ dst) {
-  constexpr TypeInfo ti = type_info(TYPE);
-  __shared__ __align__(16) uint8_t stage[64 * ti.ts];
-  const int64_t total = n * nb;
-  const int64_t i0 = (int64_t)blockIdx.x * 64;
-  const int64_t i = i0 + threadIdx.x;
-  if (i < total) {
-    const int64_t row = i / nb, b = i - row * nb;
-    float x[ti.bs];
-    if constexpr (FP8) {
-      const uint8_t *p = static_cast<const uint8_t *>(src) + row * ld + b * ti.bs;
-      if constexpr (VEC) {
-#pragma unroll
-        for (int c = 0; c < ti.bs / 16; ++c) {
-          const uint4 v = reinterpret_cast<const uint4 *>(p)[c];
-          const uint32_t wd[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-          for (int j = 0; j < 16; ++j) x[16 * c + j] = e4m3_to_f32((uint8_t)(wd[j >> 2] >> (8 * (j & 3)))) * scale;
-        }
-      } else {
-        for (int j = 0; j < ti.bs; ++j) x[j] = e4m3_to_f32(p[j]) * scale;
-      }
-    } else {
-      const float *p = static_cast<const float *>(src) + row * ld + b * ti.bs;
-      if constexpr (VEC) {
-#pragma unroll
-        for (int c = 0; c < ti.bs / 4; ++c) {
-          const float4 v = reinterpret_cast<const float4 *>(p)[c];
-          x[4 * c] = v.x;
-          x[4 * c + 1] = v.y;
-          x[4 * c + 2] = v.z;
-          x[4 * c + 3] = v.w;
-        }
-      } else {
-        for (int j = 0; j < ti.bs; ++j) x[j] = p[j];
-      }
-    }
-    uint8_t o[ti.ts];
-    quant_block<TYPE>(x, o);
-    for (int j = 0; j < ti.ts; ++j) stage[threadIdx.x * ti.ts + j] = o[j];
-  }
-  __syncthreads();
-  // blocks i0 .. i0 + nblk - 1 are bytes i0 * ts .. of dst (i0 * ts is a
-  // multiple of 64 * ts, so 16-byte aligned in the 256-byte aligned buffer)
-  const int64_t nblk = total - i0 < 64 ? total - i0 : 64;
-  const int bytes = (int)nblk * ti.ts;
-  uint8_t *q = dst + i0 * ti.ts;
-  const int whole = bytes & ~15;
-  for (int o = 16 * (int)threadIdx.x; o < whole; o += 16 * 64)
-    *reinterpret_cast<uint4 *>(q + o) = *reinterpret_cast<const uint4 *>(stage + o);
-  for (int o = whole + (int)threadIdx.x; o < bytes; o += 64) q[o] = stage[o];
 }
 
 // A block image's bytes [OFF, OFF + 4) as a little-endian word (constant
@@ -662,6 +391,15 @@ __device__ __forceinline__ void store_field(uint8_t *tiled, const Geo &g, int64_
 // and no repack pass (the repack reads these 18-34-byte blocks 2 bytes at a
 // time).
 constexpr int kQtBlocks = 4;
+
+template <int TYPE>
+__device__ __forceinline__ void quant_block(const float *x, uint8_t *o) {
+  if constexpr (TYPE == Q4_0) q_q4_0(x, o);
+  else if constexpr (TYPE == Q4_1) q_q4_1(x, o);
+  else if constexpr (TYPE == Q5_0) q_q5_0(x, o);
+  else if constexpr (TYPE == Q5_1) q_q5_1(x, o);
+  else q_q8_0(x, o);
+}
 
 template <int TYPE, bool FP8, bool VEC>
 __global__ __launch_bounds__(64) void quantize_tiled_kernel(const void *__restrict__ src, int64_t ld, Geo g,
@@ -718,54 +456,337 @@ __global__ __launch_bounds__(64) void quantize_tiled_kernel(const void *__restri
   }
 }
 
+// ------------------------------------------------------------- k-quant blocks
+// Each thread quantizes one sub-block and the super-block's 8 (Q4_K, Q5_K) or
+// 16 lanes share the rest: the largest scale by lane exchanges, packed words
+// or-ed across the lanes that hold their other bits, and every 16-byte chunk
+// stored by one lane straight into the device layout (rows past n as zeros).
+// With one thread a super-block (the values, quants and search candidates in
+// private memory, raw blocks to a staging buffer, then a repack pass) Q4_K
+// [21504, 3072] took 1022 + 39 us, now 640 (VALU-bound: about 430 operations a
+// value at one per lane and cycle); [8192, 3072] whole calls, before -> now:
+// Q2_K 496 -> 242 us, Q3_K 428 -> 133, Q4_K 567 -> 298, Q5_K 538 -> 247, Q6_K
+// 383 -> 182.
+
+// v combined over the W lanes of a super-block by or / by maximum (values never NaN there).
+template <int W>
+__device__ __forceinline__ uint32_t group_or(uint32_t v) {
+#pragma unroll
+  for (int m = 1; m < W; m *= 2) v |= (uint32_t)__shfl_xor((int)v, m);
+  return v;
+}
+template <int W>
+__device__ __forceinline__ float group_max0(float v) {
+  v = v > 0.f ? v : 0.f;  // ggml: max = 0; if (v > max) max = v
+#pragma unroll
+  for (int m = 1; m < W; m *= 2) {
+    const float u = __shfl_xor(v, m);
+    v = u > v ? u : v;
+  }
+  return v;
+}
+// The value of largest magnitude over the group's 16 lanes, the lowest lane's
+// on a tie (0 if every magnitude is 0 or NaN).
+__device__ __forceinline__ float group_absmax(float v, float &amax) {
+  float a = fabsf(v);
+  if (!(a > 0.f)) { a = 0.f; v = 0.f; }
+  int at = threadIdx.x & 15;
+#pragma unroll
+  for (int m = 1; m < 16; m *= 2) {
+    const float ua = __shfl_xor(a, m), uv = __shfl_xor(v, m);
+    const int ut = __shfl_xor(at, m);
+    if (ua > a || (ua == a && ut < at)) { a = ua; v = uv; at = ut; }
+  }
+  amax = a;
+  return v;
+}
+
+// Words of 4 quants, one per byte.
+template <int N>
+__device__ __forceinline__ void pack_bytes(const int (&L)[N], uint32_t (&p)[N / 4]) {
+#pragma unroll
+  for (int i = 0; i < N / 4; ++i)
+    p[i] = (uint32_t)L[4 * i] | ((uint32_t)L[4 * i + 1] << 8) | ((uint32_t)L[4 * i + 2] << 16) |
+           ((uint32_t)L[4 * i + 3] << 24);
+}
+// p |= the lanes' at distance m, each lane's already shifted to its bits.
+template <int N>
+__device__ __forceinline__ void or_lanes(uint32_t (&p)[N], int m) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) p[i] |= (uint32_t)__shfl_xor((int)p[i], m);
+}
+__device__ __forceinline__ void put_chunk(uint8_t *tiled, int64_t plane, int nchunks, int64_t tb, int c, int r,
+                                          const uint32_t *w) {
+  *reinterpret_cast<uint4 *>(tiled + plane + ((tb * nchunks + c) * kRowTile + r) * 16) =
+      make_uint4(w[0], w[1], w[2], w[3]);
+}
+template <typename V>
+__device__ __forceinline__ void put_record(uint8_t *tiled, int64_t plane, int size, int64_t tb, int r, int off, V v) {
+  *reinterpret_cast<V *>(tiled + plane + (tb * kRowTile + r) * size + off) = v;
+}
+
+template <int TYPE>
+constexpr int kq_lanes() {
+  return TYPE == Q4_K || TYPE == Q5_K ? 8 : 16;
+}
+
+// Sub-block j of block tb, tile row r, from its values x (`real`: a row of the
+// tensor; padding rows are zero bytes).  Every lane of the wave joins.
+template <int TYPE, int N>
+__device__ __forceinline__ void quantize_sub(const float (&x)[N], bool real, int j, uint8_t *t, const Geo &g, int64_t tb,
+                                             int r) {
+  int L[N];
+  uint32_t p[N / 4];
+  if constexpr (TYPE == Q4_K || TYPE == Q5_K) {
+    constexpr bool FIVE = TYPE == Q5_K;
+    constexpr int nmax = FIVE ? 31 : 15;
+    float w[N], sum_x2 = 0;
+#pragma unroll
+    for (int l = 0; l < N; ++l) sum_x2 += x[l] * x[l];
+    const float av_x = sqrtf(sum_x2 / 32);
+#pragma unroll
+    for (int l = 0; l < N; ++l) w[l] = av_x + fabsf(x[l]);
+    const Qkx2 s = qkx2<N, false>(nmax, x, w, FIVE ? -0.5f : -1.f, 0.1f, FIVE ? 15 : 20);
+    const float max_scale = group_max0<8>(s.scale), max_min = group_max0<8>(s.the_min);
+    const float inv_scale = max_scale > 0 ? 63.f / max_scale : 0.f;
+    const float inv_min = max_min > 0 ? 63.f / max_min : 0.f;
+    const uint32_t ls = mn<uint8_t>(63, (uint8_t)nearest_int(inv_scale * s.scale));
+    const uint32_t lm = mn<uint8_t>(63, (uint8_t)nearest_int(inv_min * s.the_min));
+    // byte j of words 0 / 1: the low 6 bits for j < 4; nibbles in word 2 and the
+    // top 2 bits above words 0 / 1's for j >= 4
+    const int sh = 8 * (j & 3);
+    const uint32_t s0 = group_or<8>((j < 4 ? ls : (ls >> 4) << 6) << sh);
+    const uint32_t s1 = group_or<8>((j < 4 ? lm : (lm >> 4) << 6) << sh);
+    const uint32_t s2 = group_or<8>(j < 4 ? 0u : ((ls & 0xF) | ((lm & 0xF) << 4)) << sh);
+    const uint16_t dh = f2h(max_scale / 63.f), mh = f2h(max_min / 63.f);
+    const float d = h2f(dh) * (float)ls, dm = h2f(mh) * (float)lm;
+    if (d) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) L[i] = mx(0, mn(nmax, nearest_int((x[i] + dm) / d)));
+    } else {  // the search's quants stay
+#pragma unroll
+      for (int i = 0; i < N; ++i) L[i] = mx(0, mn(nmax, nearest_int(s.best_iscale * (x[i] - s.best_min))));
+    }
+    pack_bytes(L, p);
+    if constexpr (FIVE) {
+      uint32_t hb[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        hb[i] = ((p[i] >> 4) & 0x01010101u) << j;
+        p[i] &= 0x0F0F0F0Fu;
+      }
+      or_lanes(hb, 1);
+      or_lanes(hb, 2);
+      or_lanes(hb, 4);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) hb[i] = real ? hb[i] : 0u;
+      if (j < 2) put_chunk(t, g.plane[2], 2, tb, j, r, j == 0 ? hb : hb + 4);
+    }
+    // sub-blocks 2g and 2g + 1 are the low and high nibbles of bytes 32 g ..
+#pragma unroll
+    for (int i = 0; i < 8; ++i) p[i] <<= 4 * (j & 1);
+    or_lanes(p, 1);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) p[i] = real ? p[i] : 0u;
+    put_chunk(t, g.plane[FIVE ? 3 : 2], 8, tb, j, r, (j & 1) == 0 ? p : p + 4);
+    if (j == 0) {
+      put_record<uint32_t>(t, g.plane[0], 4, tb, r, 0, real ? (uint32_t)dh | ((uint32_t)mh << 16) : 0u);
+      put_record<uint32_t>(t, g.plane[1], 12, tb, r, 0, real ? s0 : 0u);
+      put_record<uint32_t>(t, g.plane[1], 12, tb, r, 4, real ? s1 : 0u);
+      put_record<uint32_t>(t, g.plane[1], 12, tb, r, 8, real ? s2 : 0u);
+    }
+  } else {
+    // sub-block j = 8 H + 2 p + half: elements 128 H + 32 p + 16 half ..
+    const int H = j >> 3, pp = (j >> 1) & 3, half = j & 1;
+    if constexpr (TYPE == Q2_K) {
+      float w[N];
+#pragma unroll
+      for (int l = 0; l < N; ++l) w[l] = fabsf(x[l]);
+      const Qkx2 s = qkx2<N, true>(3, x, w, -0.5f, 0.1f, 15);
+      const float max_scale = group_max0<16>(s.scale), max_min = group_max0<16>(s.the_min);
+      uint32_t sc = 0;
+      uint16_t dh = f2h(0.f), mh = f2h(0.f);
+      if (max_scale > 0) {
+        const float iscale = 15.f / max_scale;
+        sc = (uint8_t)nearest_int(iscale * s.scale);
+        dh = f2h(max_scale / 15.f);
+      }
+      if (max_min > 0) {
+        const float iscale = 15.f / max_min;
+        sc |= (uint8_t)(nearest_int(iscale * s.the_min) << 4);
+        mh = f2h(max_min / 15.f);
+      }
+      const float d = h2f(dh) * (float)(sc & 0xF), dm = h2f(mh) * (float)(sc >> 4);
+      if (d) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) L[i] = mx(0, mn(3, nearest_int((x[i] + dm) / d)));
+      } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) L[i] = mx(0, mn(3, nearest_int(s.best_iscale * (x[i] - s.best_min))));
+      }
+      pack_bytes(L, p);
+      put_record<uint8_t>(t, g.plane[0], 16, tb, r, j, real ? (uint8_t)sc : 0);
+      if (j == 0) put_record<uint32_t>(t, g.plane[2], 4, tb, r, 0, real ? (uint32_t)dh | ((uint32_t)mh << 16) : 0u);
+    } else if constexpr (TYPE == Q3_K) {
+      float amax;
+      const float scale = q3_group<N>(4, x, L);
+      const float max_scale = group_absmax(scale, amax);
+      uint32_t l6 = 0;
+      uint16_t dh = f2h(0.f);
+      if (max_scale) {
+        const float iscale = -32.f / max_scale;
+        const int8_t l = (int8_t)nearest_int(iscale * scale);
+        l6 = (uint32_t)(mx(-32, mn(31, (int)l)) + 32);
+        dh = f2h(1 / iscale);
+      }
+      const uint32_t low = (l6 & 0xF) << (8 * (j & 3) + 4 * (j >> 3));
+      const uint32_t s0 = group_or<16>((j & 4) ? 0u : low), s1 = group_or<16>((j & 4) ? low : 0u);
+      const uint32_t s2 = group_or<16>((l6 >> 4) << (8 * (j & 3) + 2 * (j >> 2)));
+      // without a scale the 12 bytes are zero, which reads back as -32
+      const float d = h2f(dh) * (float)((int)l6 - 32);
+      if (d) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) L[i] = mx(-4, mn(3, nearest_int(x[i] / d))) + 4;
+      }
+      uint32_t hm[4];
+      pack_bytes(L, p);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        hm[i] = ((p[i] >> 2) & 0x01010101u) << (j >> 1);  // bit 4 H + p: the value is above 3
+        p[i] &= 0x03030303u;
+      }
+      or_lanes(hm, 2);
+      or_lanes(hm, 4);
+      or_lanes(hm, 8);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) hm[i] = real ? hm[i] : 0u;
+      if (j < 2) put_chunk(t, g.plane[0], 2, tb, j, r, hm);
+      if (j == 0) {
+        put_record<uint32_t>(t, g.plane[2], 12, tb, r, 0, real ? s0 : 0u);
+        put_record<uint32_t>(t, g.plane[2], 12, tb, r, 4, real ? s1 : 0u);
+        put_record<uint32_t>(t, g.plane[2], 12, tb, r, 8, real ? s2 : 0u);
+        put_record<uint16_t>(t, g.plane[3], 2, tb, r, 0, real ? dh : 0);
+      }
+    } else {
+      static_assert(TYPE == Q6_K);
+      float best_iscale, amax;
+      bool zero;
+      const float scale = qx_rmse1<N>(32, x, best_iscale, zero);
+      const float max_scale = group_absmax(scale, amax);
+      const bool none = amax < kGroupMaxEps;  // a super-block of zeros is zero bytes
+      const float iscale = -128.f / max_scale;
+      const uint16_t dh = none ? f2h(0.f) : f2h(1 / iscale);
+      const int sc = none ? 0 : (int)(int8_t)mn(127, nearest_int(iscale * scale));
+      const float d = h2f(dh) * (float)sc;
+      if (d) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) L[i] = mx(-32, mn(31, nearest_int(x[i] / d))) + 32;
+      } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) L[i] = zero || none ? 0 : 32 + mx(-32, mn(31, nearest_int(best_iscale * x[i])));
+      }
+      uint32_t ph[4];
+      pack_bytes(L, p);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        ph[i] = ((p[i] >> 4) & 0x03030303u) << (2 * pp);
+        p[i] = (p[i] & 0x0F0F0F0Fu) << (4 * (pp >> 1));
+      }
+      or_lanes(ph, 2);
+      or_lanes(ph, 4);
+      or_lanes(p, 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        p[i] = real ? p[i] : 0u;
+        ph[i] = real ? ph[i] : 0u;
+      }
+      if (pp < 2) put_chunk(t, g.plane[0], 8, tb, 4 * H + 2 * pp + half, r, p);
+      if (pp == 0) put_chunk(t, g.plane[1], 4, tb, 2 * H + half, r, ph);
+      put_record<uint8_t>(t, g.plane[2], 16, tb, r, j, real ? (uint8_t)sc : 0);
+      if (j == 0) put_record<uint16_t>(t, g.plane[3], 2, tb, r, 0, real ? dh : 0);
+    }
+    if constexpr (TYPE == Q2_K || TYPE == Q3_K) {
+      // the 2-bit planes: byte 32 H + 16 half + i holds the four p's at bits 2 p
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p[i] <<= 2 * pp;
+      or_lanes(p, 2);
+      or_lanes(p, 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p[i] = real ? p[i] : 0u;
+      if (pp == 0) put_chunk(t, g.plane[1], 4, tb, 2 * H + half, r, p);
+    }
+  }
+}
+
+// Workgroup: 256 / lanes rows of one super-block column (columns fastest);
+// lane -> (row, sub-block), sub-block fastest.
+template <int TYPE, bool FP8, bool VEC>
+__global__ __launch_bounds__(256) void quantize_k_kernel(const void *__restrict__ src, int64_t ld, Geo g, float scale,
+                                                         uint8_t *__restrict__ tiled) {
+  constexpr int kL = kq_lanes<TYPE>(), N = 256 / kL;
+  const int j = threadIdx.x % kL;
+  const int64_t rg = blockIdx.x / (uint32_t)g.nb, b = blockIdx.x - rg * g.nb;
+  const int64_t row = rg * (256 / kL) + threadIdx.x / kL;  // < 64 ntiles
+  const bool real = row < g.n;
+  float x[N];
+  const int64_t at = (real ? row : 0) * ld + b * 256 + j * N;
+  if constexpr (FP8) {
+    const uint8_t *p = static_cast<const uint8_t *>(src) + at;
+    if constexpr (VEC) {
+#pragma unroll
+      for (int c = 0; c < N / 16; ++c) {
+        const uint4 v = reinterpret_cast<const uint4 *>(p)[c];
+        const uint32_t wd[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[16 * c + i] = e4m3_to_f32((uint8_t)(wd[i >> 2] >> (8 * (i & 3)))) * scale;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < N; ++i) x[i] = e4m3_to_f32(p[i]) * scale;
+    }
+  } else {
+    const float *p = static_cast<const float *>(src) + at;
+    if constexpr (VEC) {
+#pragma unroll
+      for (int c = 0; c < N / 4; ++c) {
+        const float4 v = reinterpret_cast<const float4 *>(p)[c];
+        x[4 * c] = v.x;
+        x[4 * c + 1] = v.y;
+        x[4 * c + 2] = v.z;
+        x[4 * c + 3] = v.w;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < N; ++i) x[i] = p[i];
+    }
+  }
+  quantize_sub<TYPE, N>(x, real, j, tiled, g, (row / kRowTile) * g.nb + b, (int)(row % kRowTile));
+}
+
 template <bool FP8>
-hipError_t launch_quantize_tiled_src(int type, const void *src, int64_t ld, float scale, void *tiled, const Geo &g,
+hipError_t launch_quantize_src(int type, const void *src, int64_t ld, float scale, void *tiled, const Geo &g,
                                      hipStream_t stream) {
   if (g.n == 0 || g.nb == 0) return hipSuccess;
   const int64_t es = FP8 ? 1 : 4;
   const bool vec = (reinterpret_cast<uintptr_t>(src) & 15) == 0 && (ld * es) % 16 == 0;
-  const dim3 grid((unsigned)((g.nb + kQtBlocks - 1) / kQtBlocks), (unsigned)g.ntiles);
-  bool ok = false;
-  auto go = [&]<int T>() {
-    if (vec)
-      hipLaunchKernelGGL((quantize_tiled_kernel<T, FP8, true>), grid, dim3(64), 0, stream, src, ld, g, scale,
-                         static_cast<uint8_t *>(tiled));
-    else
-      hipLaunchKernelGGL((quantize_tiled_kernel<T, FP8, false>), grid, dim3(64), 0, stream, src, ld, g, scale,
-                         static_cast<uint8_t *>(tiled));
-    ok = true;
-  };
-  switch (type) {
-    case Q4_0: go.template operator()<Q4_0>(); break;
-    case Q4_1: go.template operator()<Q4_1>(); break;
-    case Q5_0: go.template operator()<Q5_0>(); break;
-    case Q5_1: go.template operator()<Q5_1>(); break;
-    case Q8_0: go.template operator()<Q8_0>(); break;
-    default: break;
-  }
-  if (!ok) return hipErrorInvalidValue;
-  return hipGetLastError();
-}
-
-template <bool FP8>
-hipError_t launch_quantize_src(int type, const void *src, int64_t ld, int64_t n, int64_t k, float scale,
-                               void *dst_raw, hipStream_t stream) {
-  const TypeInfo ti = type_info(type);
-  const int64_t nb = k / ti.bs;
-  const int64_t total = n * nb;
-  if (total == 0) return hipSuccess;
-  if ((reinterpret_cast<uintptr_t>(dst_raw) & 15) != 0) return hipErrorInvalidValue;
-  // 16-byte source loads need every block's first element 16-byte aligned
-  const int64_t es = FP8 ? 1 : 4;
-  const bool vec = (reinterpret_cast<uintptr_t>(src) & 15) == 0 && (ld * es) % 16 == 0 && (ti.bs * es) % 16 == 0;
-  const unsigned grid = (unsigned)((total + 63) / 64);
   bool ok = dispatch_type(type, [&]<int T>() {
-    if (vec)
-      hipLaunchKernelGGL((quantize_kernel<T, FP8, true>), dim3(grid), dim3(64), 0, stream, src, ld, n, nb, scale,
-                         static_cast<uint8_t *>(dst_raw));
-    else
-      hipLaunchKernelGGL((quantize_kernel<T, FP8, false>), dim3(grid), dim3(64), 0, stream, src, ld, n, nb, scale,
-                         static_cast<uint8_t *>(dst_raw));
+    if constexpr (type_info(T).bs == 32) {
+      const dim3 grid((unsigned)((g.nb + kQtBlocks - 1) / kQtBlocks), (unsigned)g.ntiles);
+      if (vec)
+        hipLaunchKernelGGL((quantize_tiled_kernel<T, FP8, true>), grid, dim3(64), 0, stream, src, ld, g, scale,
+                           static_cast<uint8_t *>(tiled));
+      else
+        hipLaunchKernelGGL((quantize_tiled_kernel<T, FP8, false>), grid, dim3(64), 0, stream, src, ld, g, scale,
+                           static_cast<uint8_t *>(tiled));
+    } else {
+      const dim3 grid((unsigned)(g.nb * (g.ntiles * kRowTile * kq_lanes<T>() / 256)));
+      if (vec)
+        hipLaunchKernelGGL((quantize_k_kernel<T, FP8, true>), grid, dim3(256), 0, stream, src, ld, g, scale,
+                           static_cast<uint8_t *>(tiled));
+      else
+        hipLaunchKernelGGL((quantize_k_kernel<T, FP8, false>), grid, dim3(256), 0, stream, src, ld, g, scale,
+                           static_cast<uint8_t *>(tiled));
+    }
   });
   if (!ok) return hipErrorInvalidValue;
   return hipGetLastError();
@@ -773,22 +794,10 @@ hipError_t launch_quantize_src(int type, const void *src, int64_t ld, int64_t n,
 
 }  // namespace
 
-hipError_t launch_quantize(int type, const float *src, int64_t ld, int64_t n, int64_t k, void *dst_raw,
+hipError_t launch_quantize(int type, const void *src, bool fp8, int64_t ld, float scale, void *tiled, const Geo &g,
                            hipStream_t stream) {
-  return launch_quantize_src<false>(type, src, ld, n, k, 1.0f, dst_raw, stream);
-}
-
-hipError_t launch_quantize_fp8(int type, const uint8_t *src, int64_t ld, int64_t n, int64_t k, float scale,
-                               void *dst_raw, hipStream_t stream) {
-  return launch_quantize_src<true>(type, src, ld, n, k, scale, dst_raw, stream);
-}
-
-bool quantize_tiled_ok(int type) { return type == Q4_0 || type == Q4_1 || type == Q5_0 || type == Q5_1 || type == Q8_0; }
-
-hipError_t launch_quantize_tiled(int type, const void *src, bool fp8, int64_t ld, float scale, void *tiled,
-                                 const Geo &g, hipStream_t stream) {
-  return fp8 ? launch_quantize_tiled_src<true>(type, src, ld, scale, tiled, g, stream)
-             : launch_quantize_tiled_src<false>(type, src, ld, 1.0f, tiled, g, stream);
+  return fp8 ? launch_quantize_src<true>(type, src, ld, scale, tiled, g, stream)
+             : launch_quantize_src<false>(type, src, ld, 1.0f, tiled, g, stream);
 }
 
 }  // namespace mq
