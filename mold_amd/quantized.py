@@ -56,15 +56,28 @@ QUANT_TYPES = [GgmlDType.Q4_0, GgmlDType.Q4_1, GgmlDType.Q5_0, GgmlDType.Q5_1, G
                GgmlDType.Q2_K, GgmlDType.Q3_K, GgmlDType.Q4_K, GgmlDType.Q5_K, GgmlDType.Q6_K]
 
 
+_TORCH = None
+
+
 def _torch():
-    import torch
-    return torch
+    """torch, imported on first use (an import statement per call costs as much as
+    the argument checks of a GEMV)."""
+    global _TORCH
+    if _TORCH is None:
+        import torch
+        _TORCH = torch
+    return _TORCH
 
 
 def _stream_ptr(stream=None) -> int:
+    """The hipStream_t of `stream`, or of torch's current stream on the current device
+    (read as a pointer: making the Stream object takes 2.7 us of a 13 us GEMV call)."""
+    if stream is not None:
+        return int(stream.cuda_stream)
     torch = _torch()
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return int(s.cuda_stream)
+    if torch.cuda.is_initialized():
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return int(torch.cuda.current_stream().cuda_stream)
 
 
 class Device:
@@ -110,7 +123,17 @@ class Device:
             pass
 
 
+_DTYPE_CODES: Dict[object, int] = {}
+
+
 def _dtype_code(dt) -> int:
+    code = _DTYPE_CODES.get(dt)
+    if code is None:
+        code = _DTYPE_CODES[dt] = _dtype_code_of(dt)
+    return code
+
+
+def _dtype_code_of(dt) -> int:
     torch = _torch()
     if dt in (torch.float32, "f32", GgmlDType.F32):
         return int(GgmlDType.F32)
@@ -248,47 +271,45 @@ class QMatMul:
         """y = act(x . W^T + bias); with act_from > 0 the activation applies to output
         columns act_from .. n-1 only (mq_qmatmul_act_from)."""
         torch = _torch()
-        n, k = self.w.shape
+        w = self.w
+        n, k = w.shape
         if not 0 <= act_from <= n:
             raise ValueError(f"QMatMul: act_from {act_from} outside 0 .. {n}")
-
-        def call(xp, xt, m, ldx, y, yt, ldy, b):
-            lib = _lib.load()
-            if act_from:
-                return lib.mq_qmatmul_act_from(self.w.device.handle, self.w.handle, xp, xt, m, ldx, y, yt, ldy, b,
-                                               int(act), int(act_from), _stream_ptr(stream))
-            return lib.mq_qmatmul(self.w.device.handle, self.w.handle, xp, xt, m, ldx, y, yt, ldy, b, int(act),
-                                  _stream_ptr(stream))
         if isinstance(x, Q8KActivations):
             if x.k != k:
                 raise ValueError(f"QMatMul: x k {x.k} != weight k {k}")
             out_dtype = out_dtype or (out.dtype if out is not None else torch.float32)
-            if out is None:
-                out = torch.empty((x.m, n), dtype=out_dtype, device=x.data.device)
-            assert out.dtype == out_dtype and tuple(out.shape) == (x.m, n)
-            if bias is not None:
-                assert bias.dtype == torch.float32 and bias.is_contiguous() and bias.numel() == n
-            check(call(x.data.data_ptr(), _lib.MQ_X_Q8K, x.m, k, out.data_ptr(), _dtype_code(out_dtype), out.stride(0),
-                       bias.data_ptr() if bias is not None else None))
-            return out.reshape(*x.lead, n)
-        if x.shape[-1] != k:
-            raise ValueError(f"QMatMul: x last dim {x.shape[-1]} != weight k {k}")
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, k)
-        if x2.stride(1) != 1:
-            x2 = x2.contiguous()
-        m = x2.shape[0]
-        if out_dtype is None:
-            out_dtype = out.dtype if out is not None else x.dtype
+            lead, m, x_code, ldx, x_data = x.lead, x.m, _lib.MQ_X_Q8K, k, x.data
+        else:
+            if x.shape[-1] != k:
+                raise ValueError(f"QMatMul: x last dim {x.shape[-1]} != weight k {k}")
+            lead = x.shape[:-1]
+            x_data = x if len(lead) == 1 else x.reshape(-1, k)
+            if x_data.stride(1) != 1:
+                x_data = x_data.contiguous()
+            m, ldx = x_data.shape[0], x_data.stride(0)
+            if out_dtype is None:
+                out_dtype = out.dtype if out is not None else x.dtype
+            x_code = _dtype_code(x_data.dtype)
         if out is None:
-            out = torch.empty((m, n), dtype=out_dtype, device=x.device)
+            out = torch.empty((m, n), dtype=out_dtype, device=x_data.device)
         else:
             assert out.dtype == out_dtype and tuple(out.shape) == (m, n)
+        b = None
         if bias is not None:
             assert bias.dtype == torch.float32 and bias.is_contiguous() and bias.numel() == n
-        check(call(x2.data_ptr(), _dtype_code(x2.dtype), m, x2.stride(0), out.data_ptr(), _dtype_code(out_dtype),
-                   out.stride(0), bias.data_ptr() if bias is not None else None))
-        return out.reshape(*lead, n)
+            b = bias.data_ptr()
+        lib = _lib.load()
+        y_code = _dtype_code(out_dtype)
+        if act_from:
+            rc = lib.mq_qmatmul_act_from(w.device.handle, w.handle, x_data.data_ptr(), x_code, m, ldx, out.data_ptr(), y_code,
+                                         out.stride(0), b, int(act), int(act_from), _stream_ptr(stream))
+        else:
+            rc = lib.mq_qmatmul(w.device.handle, w.handle, x_data.data_ptr(), x_code, m, ldx, out.data_ptr(), y_code,
+                                out.stride(0), b, int(act), _stream_ptr(stream))
+        if rc:
+            check(rc)
+        return out if len(lead) == 1 else out.reshape(*lead, n)
 
     __call__ = forward
 
