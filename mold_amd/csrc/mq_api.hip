@@ -201,8 +201,18 @@ struct Plan {
   size_t total = 0;
 };
 
+// Whether y's rows touch f32 x's memory: such a call stages x first (a copy made
+// before any y is written), as a kernel that reads f32 x in place could not.
+bool y_over_x(const mq_qtensor *w, const void *x, int64_t m, int64_t ldx, const void *y, int y_dtype, int64_t ldy) {
+  const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), y0 = reinterpret_cast<uintptr_t>(y);
+  const uintptr_t xb = (uintptr_t)((m - 1) * ldx + w->k) * 4;
+  const uintptr_t yb = (uintptr_t)((m - 1) * ldy + w->n) * (y_dtype == MQ_F32 ? 4 : 2);
+  return x0 < y0 + yb && y0 < x0 + xb;
+}
+
+// f32_in_place: the few-rows kernel may read f32 x where it lies.
 Plan plan_qmatmul(const mq_ctx *ctx, const mq_qtensor *w, const void *x, int x_dtype, int64_t m, int64_t ldx,
-                  bool gated, bool tail_split = true) {
+                  bool gated, bool tail_split = true, bool f32_in_place = true) {
   Plan p;
   const int64_t n = w->n, k = w->k;
   if (m <= kGemvMaxM && !gated) {
@@ -213,12 +223,21 @@ Plan plan_qmatmul(const mq_ctx *ctx, const mq_qtensor *w, const void *x, int x_d
     p.stage_bytes = p.stage_gemv ? (size_t)m * k * sizeof(float) : 0;
   } else {
     p.kp = (k + 63) / 64 * 64;
-    p.stage_gemm =
-        !(x_dtype == MQ_BF16 && k == p.kp && (ldx % 8) == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0);
+    const bool aligned = (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+    p.stage_gemm = !(x_dtype == MQ_BF16 && k == p.kp && (ldx % 8) == 0 && aligned);
+    bool few = gemm_skinny_ok(w->dtype, m, n, k, tail_split);
+    if (few) {
+      p.tail = gemm_skinny_plan(m, n, k, ctx->cu_count, tail_split);
+      if (x_dtype == MQ_F32 && f32_in_place && aligned && ldx % 4 == 0 && gemm_skinny_reads_f32(w->dtype, n, k, p.tail))
+        p.stage_gemm = false;
+      // its byte offsets into x are 31 bits
+      few = m * (p.stage_gemm ? p.kp : ldx) * 4 < (int64_t(1) << 31);
+      if (!few) p.stage_gemm = p.stage_gemm || x_dtype == MQ_F32;
+    }
     const int64_t lda = p.stage_gemm ? p.kp : ldx;
     p.stage_bytes = p.stage_gemm ? (size_t)m * p.kp * sizeof(__bf16) : 0;
-    p.tail = gemm_tail_plan(w->dtype, m, n, k, ctx->cu_count, tail_split);
-    if (p.tail.kparts > 1 && gemm_fast_ok(w->dtype, m, k, lda)) p.part_bytes = gemm_tail_bytes(p.tail, m, n);
+    if (!few) p.tail = gemm_tail_plan(w->dtype, m, n, k, ctx->cu_count, tail_split);
+    if (p.tail.kparts > 1 && (few || gemm_fast_ok(w->dtype, m, k, lda))) p.part_bytes = gemm_tail_bytes(p.tail, m, n);
     else p.tail.kparts = 1;
   }
   p.part_off = align256(p.stage_bytes);
@@ -257,16 +276,18 @@ int run_qmatmul(mq_ctx *ctx, const mq_qtensor *w, const Plan &p, uint8_t *ws, co
     if (e != hipSuccess) return hip_fail(e, "gemv launch");
     return MQ_OK;
   }
-  const __bf16 *a = static_cast<const __bf16 *>(x);
+  const void *a = x;
+  int at = x_dtype;
   int64_t lda = ldx;
   if (p.stage_gemm) {
     __bf16 *st = reinterpret_cast<__bf16 *>(ws + p.stage_off);
     hipError_t e = launch_stage_bf16(x, x_dtype, m, k, ldx, st, p.kp, s);
     if (e != hipSuccess) return hip_fail(e, "stage activations");
     a = st;
+    at = MQ_BF16;
     lda = p.kp;
   }
-  hipError_t e = launch_gemm(w->dtype, wv, n, k, w->geo.ntiles, a, m, lda, y, y_dtype, ldy, bias, gate, act, p.tail,
+  hipError_t e = launch_gemm(w->dtype, wv, n, k, w->geo.ntiles, a, at, m, lda, y, y_dtype, ldy, bias, gate, act, p.tail,
                              partial, s);
   if (e != hipSuccess) return hip_fail(e, "gemm launch");
   return MQ_OK;
@@ -810,10 +831,12 @@ int mq_qmatmul_workspace_size(mq_ctx *ctx, const mq_qtensor *w, int x_dtype, int
   if (is_dense(w->dtype))
     return fail(MQ_E_UNSUPPORTED, "mq_qmatmul_workspace_size: dense %s weights take no quantized matmul",
                 dense_name(w->dtype));
-  // a misaligned x pointer takes every staging path, so this is the bound
-  // over all x placements and strides
+  // a misaligned x pointer takes every staging path and an aligned one the
+  // few-rows kernel's K split, so this is the bound over all x placements and
+  // strides
   const void *worst = reinterpret_cast<const void *>(uintptr_t(1));
-  *bytes = m == 0 ? 0 : plan_qmatmul(ctx, w, worst, x_dtype, m, w->k, gated != 0).total;
+  *bytes = m == 0 ? 0 : std::max(plan_qmatmul(ctx, w, worst, x_dtype, m, w->k, gated != 0).total,
+                                 plan_qmatmul(ctx, w, nullptr, x_dtype, m, w->k, gated != 0).total);
   return MQ_OK;
 }
 
@@ -825,7 +848,8 @@ static int qmatmul_cols(const char *fn, mq_ctx *ctx, const mq_qtensor *w, const 
   if (rc || m == 0) return rc;
   DeviceGuard g(ctx->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const Plan p = plan_qmatmul(ctx, w, x, x_dtype, m, ldx, false, tail_split_on(ctx, s));
+  const Plan p = plan_qmatmul(ctx, w, x, x_dtype, m, ldx, false, tail_split_on(ctx, s),
+                              x_dtype != MQ_F32 || !y_over_x(w, x, m, ldx, y, y_dtype, ldy));
   uint8_t *ws = nullptr;
   if (p.total) {
     rc = stream_workspace(ctx, s, p.total, &ws);
@@ -873,7 +897,8 @@ int mq_qmatmul_noalloc(mq_ctx *ctx, const mq_qtensor *w, const void *x, int x_dt
   if (rc || m == 0) return rc;
   DeviceGuard g(ctx->device);
   const Plan p =
-      plan_qmatmul(ctx, w, x, x_dtype, m, ldx, false, tail_split_on(ctx, static_cast<hipStream_t>(stream)));
+      plan_qmatmul(ctx, w, x, x_dtype, m, ldx, false, tail_split_on(ctx, static_cast<hipStream_t>(stream)),
+                   x_dtype != MQ_F32 || !y_over_x(w, x, m, ldx, y, y_dtype, ldy));
   if (p.total > MQ_NOALLOC_SCRATCH_BYTES)
     return fail(MQ_E_INVALID,
                 "mq_qmatmul_noalloc: this call needs %zu bytes of scratch, more than its fixed %zu bytes "
@@ -895,7 +920,8 @@ int mq_qmatmul_gated_add(mq_ctx *ctx, const mq_qtensor *w, const void *x, int x_
   DeviceGuard g(ctx->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
   // every m takes the GEMM kernel: its epilogue holds the gated update
-  const Plan p = plan_qmatmul(ctx, w, x, x_dtype, m, ldx, true, tail_split_on(ctx, s));
+  const Plan p = plan_qmatmul(ctx, w, x, x_dtype, m, ldx, true, tail_split_on(ctx, s),
+                              x_dtype != MQ_F32 || !y_over_x(w, x, m, ldx, y, MQ_F32, ldy));
   uint8_t *ws = nullptr;
   if (p.total) {
     rc = stream_workspace(ctx, s, p.total, &ws);

@@ -10,7 +10,7 @@
 //     is fetched once for 256 output features (against two 4-wave 256 x 128
 //     workgroups per CU: 3-8 % faster on every large BASELINE shape, same
 //     outputs); small m: 64- or 128-row tiles of 4 waves x 128 features, three
-//     or four workgroups per CU;
+//     or four workgroups per CU (gemm_skinny_kernel up to 96 rows);
 //   * wave w owns output features 32w .. 32w+31 of the tile for all its
 //     rows: lane (l32, h) decodes weight row l32 of that run straight into
 //     the MFMA B operand (per-type decoders, mq_bfrag.h), so every weight is
@@ -476,6 +476,224 @@ __global__ __launch_bounds__(64 * kW, 8 / kW) void gemm_fast_kernel(
   }
 }
 
+// Few rows (m <= 96): every weight is decoded for kFM = 32 ceil(m / 32) rows
+// only, so a launch is bound by getting the weights in and decoding them, not
+// by the matrix cores.  Eight waves on 128 features: wave (f, kh) owns 32 of
+// them and half kh of each chunk of K, so two waves a SIMD decode side by side
+// and the halves are added through LDS at the end.  A chunk of kKC columns
+// (512, or 256 above 64 rows: two buffers of x must fit the LDS) is loaded
+// whole, x by LDS DMA and the wave's weights to registers, while the chunk
+// before is computed: one memory latency per chunk, where gemm_fast_kernel
+// pays one per 64 columns (77 x 4096 -> 4096 Q8_0: 14.3 us there, 12.2 here,
+// under the same trace; 9 rows 11 us and 6).
+template <int FM>
+constexpr int skinny_chunk() {
+  return FM <= 64 ? 512 : 256;
+}
+
+template <int TYPE, typename XT, typename OUT, bool GATED, int kFM>
+__global__ __launch_bounds__(512, 2) void gemm_skinny_kernel(
+    WView w, int64_t n, int64_t k, int64_t ntiles_w, const XT *__restrict__ a, int64_t m, int64_t lda, OUT *y, int64_t ldy, const float *__restrict__ bias, const float *__restrict__ gate, int act, int kparts,
+    float *__restrict__ partial) {
+  using TT = bfrag::T<TYPE>;
+  constexpr int kP = TT::kUnitK / kFK;                // K steps per weight unit
+  constexpr int kMB = kFM / 32, kKC = skinny_chunk<kFM>(), kSteps = kKC / kFK;
+  constexpr int kWS = kSteps / 2;                     // this wave's steps of a chunk
+  constexpr int kNU = kWS >= kP ? kWS / kP : 1;       // and its weight units (one may be half used)
+  constexpr bool kHalf = kWS < kP;                    // steps 2 kh, 2 kh + 1 of the chunk's one unit
+  constexpr int kDM = kFM * kSteps / 64;              // DMA loads per wave and chunk
+  constexpr int kTileBytes = kFM * kFK * 2;           // x of one step
+  __shared__ uint4 lds_a[2][kFM * kKC / 8];
+
+  const int tile = blockIdx.x / kparts, part = blockIdx.x - tile * kparts;
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), f = wave & 3, kh = wave >> 2;
+  const int64_t c0 = (int64_t)tile * 128 + 32 * f;
+  const int64_t wt_raw = c0 / kRowTile;
+  const int wrow = (int)(c0 - wt_raw * kRowTile) + l32;
+  const int64_t wt = wt_raw < ntiles_w ? wt_raw : ntiles_w - 1;  // keep reads in bounds
+  const int64_t chunks = (k + kKC - 1) / kKC;
+  const int64_t cb = part * chunks / kparts, ce = (part + 1) * chunks / kparts;
+  const int64_t units = k / TT::kUnitK;
+
+  f32x16 acc[kMB];
+#pragma unroll
+  for (int i = 0; i < kMB; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
+
+  // x of a chunk: per step a tile of kFM rows of 128 bytes, swizzled as in
+  // gemm_fast_kernel; a load fills 8 rows of one step's tile.  Wave w loads
+  // step w % kSteps, row groups w / kSteps + i * 8 / kSteps: bf16 x by LDS
+  // DMA, f32 x through registers (two 16-byte loads, rounded to bf16 into the
+  // same 16 LDS bytes), so f32 x needs no staging pass (2.7 us of a 77-row call).
+  constexpr bool kF32 = std::is_same_v<XT, float>;
+  const int step = wave % kSteps, g0 = wave / kSteps;
+  uint32_t voff[kDM];
+#pragma unroll
+  for (int i = 0; i < kDM; ++i) {
+    const int row = 8 * (g0 + i * (8 / kSteps)) + (lane >> 3);
+    const int gch = (lane & 7) ^ ((row >> 1) & 7);
+    const int64_t r = row < m ? row : m - 1;
+    voff[i] = (uint32_t)((r * lda + gch * 8) * (int)sizeof(XT));
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(&lds_a[0][0]) + (uint32_t)(step * kTileBytes + 1024 * g0);
+  float4 xr[kF32 ? kDM : 1][2];
+  auto load_x = [&](int64_t c, int buf) {
+    const int64_t kk = c * kKC + step * kFK;
+    if (kk >= k) return;  // past K (a last chunk of fewer steps): never read
+    const uint64_t g = reinterpret_cast<uint64_t>(a + kk);
+    const char *sb = reinterpret_cast<const char *>(((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(g >> 32)) << 32) |
+                                                    (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)g));
+#pragma unroll
+    for (int i = 0; i < kDM; ++i) {
+      if constexpr (kF32) {
+        xr[i][0] = *reinterpret_cast<const float4 *>(sb + voff[i]);
+        xr[i][1] = *reinterpret_cast<const float4 *>(sb + voff[i] + 16);
+      } else {
+        dma16(sb, voff[i],
+              __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)(buf * (kFM * kKC * 2) + 1024 * (8 / kSteps) * i)));
+      }
+    }
+  };
+  // f32 x: the loaded chunk into LDS (its buffer is free: every wave is past
+  // the barrier that ended its last use)
+  auto store_x = [&](int buf) {
+    if constexpr (kF32) {
+      typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
+#pragma unroll
+      for (int i = 0; i < kDM; ++i) {
+        const float4 p = xr[i][0], q = xr[i][1];
+        bf16x8 v;
+        v[0] = (__bf16)p.x; v[1] = (__bf16)p.y; v[2] = (__bf16)p.z; v[3] = (__bf16)p.w;
+        v[4] = (__bf16)q.x; v[5] = (__bf16)q.y; v[6] = (__bf16)q.z; v[7] = (__bf16)q.w;
+        *(lds_bf16x8 *)(uintptr_t)(lds0 + (uint32_t)(buf * (kFM * kKC * 2) + 1024 * (8 / kSteps) * i + 16 * lane)) = v;
+      }
+    }
+  };
+  const int swz = (l32 >> 1) & 7;
+  auto read_a = [&](int buf, int t, int mb, int S) -> bf16x8 {
+    const char *p = reinterpret_cast<const char *>(lds_a[buf]) + t * kTileBytes + l32 * 128 +
+                    ((TT::chunk(S, h) ^ swz) << 4) + mb * 4096;
+    return *reinterpret_cast<const bf16x8 *>(p);
+  };
+  // unit j of this wave in chunk c (past the last one: the last, not used)
+  auto unit_of = [&](int64_t c, int j) {
+    const int64_t u = kHalf ? c : c * (kSteps / kP) + kh * kNU + j;
+    return u < units ? u : units - 1;
+  };
+  auto load_w = [&](int64_t c, typename TT::Raw *raw) {
+#pragma unroll
+    for (int j = 0; j < kNU; ++j) {
+      const int64_t u = unit_of(c, j);
+      TT::load_prep(raw[j], w, wt, wrow, u, h);
+      if constexpr (kHalf) {
+        if (kh == 0) {
+          TT::template reload<0>(raw[j], w, wt, wrow, u, h);
+          TT::template reload<1>(raw[j], w, wt, wrow, u, h);
+        } else {
+          TT::template reload<2>(raw[j], w, wt, wrow, u, h);
+          TT::template reload<3>(raw[j], w, wt, wrow, u, h);
+        }
+      } else {
+        static_for<kP>([&]<int G>() { TT::template reload<G>(raw[j], w, wt, wrow, u, h); });
+      }
+    }
+  };
+  // NS steps from step G0 of one unit against the chunk's tiles t0 ..: the
+  // next slice's weights are decoded beside a slice's MFMAs
+  auto run_steps = [&]<int G0, int NS>(const typename TT::Raw &raw, const typename TT::Sc &sc, int buf, int t0) {
+    bf16x8 bf[2];
+    bf[0] = TT::template frag<G0, 0>(raw, sc);
+    static_for<4 * NS>([&]<int Q>() {
+      if constexpr (Q + 1 < 4 * NS) bf[(Q + 1) & 1] = TT::template frag<G0 + (Q + 1) / 4, (Q + 1) % 4>(raw, sc);
+#pragma unroll
+      for (int mb = 0; mb < kMB; ++mb)
+        acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(read_a(buf, t0 + Q / 4, mb, Q % 4), bf[Q & 1], acc[mb], 0, 0, 0);
+    });
+  };
+  auto compute = [&](int64_t c, int buf, const typename TT::Raw *raw) {
+#pragma unroll
+    for (int j = 0; j < kNU; ++j) {
+      typename TT::Sc sc;
+      TT::prep(raw[j], sc, h);
+      if constexpr (kHalf) {
+        if (kh == 0) run_steps.template operator()<0, 2>(raw[j], sc, buf, 0);
+        else run_steps.template operator()<2, 2>(raw[j], sc, buf, 2);
+      } else if (c * (kSteps / kP) + kh * kNU + j < units) {
+        run_steps.template operator()<0, kP>(raw[j], sc, buf, kh * kWS + j * kP);
+      }
+    }
+  };
+
+  typename TT::Raw raw[2][kNU];
+  load_w(cb, raw[0]);
+  load_x(cb, 0);
+  store_x(0);
+  step_barrier();
+  for (int64_t c = cb; c < ce; c += 2) {
+    if (c + 1 < ce) {
+      load_w(c + 1, raw[1]);
+      load_x(c + 1, 1);
+    }
+    compute(c, 0, raw[0]);
+    if (c + 1 >= ce) break;
+    store_x(1);
+    step_barrier();
+    if (c + 2 < ce) {
+      load_w(c + 2, raw[0]);
+      load_x(c + 2, 0);
+    }
+    compute(c + 1, 1, raw[1]);
+    if (c + 2 < ce) store_x(0);
+    step_barrier();
+  }
+  step_barrier();  // every wave is done with x: its LDS is free
+
+  // the two K halves: waves of half 1 leave their sums in LDS, half 0 adds them
+  float *red = reinterpret_cast<float *>(&lds_a[0][0]) + (f * kMB * 16) * 64 + lane;
+  if (kh == 1) {
+#pragma unroll
+    for (int mb = 0; mb < kMB; ++mb)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) red[(mb * 16 + e) * 64] = acc[mb][e];
+  }
+  __syncthreads();
+  if (kh == 1 || c0 >= n) return;
+#pragma unroll
+  for (int mb = 0; mb < kMB; ++mb)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[mb][e] += red[(mb * 16 + e) * 64];
+
+  // ---- epilogue: lane holds feature c0 + l32 of rows 32 mb + 8 (e / 4) + 4 h + e % 4
+  if (kparts > 1) {
+    float *pt = partial + ((int64_t)tile * kparts + part) * (kFM * 128) + 4 * h * 128 + 32 * f + l32;
+#pragma unroll
+    for (int mb = 0; mb < kMB; ++mb)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) pt[(mb * 32 + 8 * (e >> 2) + (e & 3)) * 128] = acc[mb][e];
+    return;
+  }
+  const int64_t col = c0 + l32;
+  if (col >= n) return;
+  const int la = act_at(act, col);
+  const float bv = bias ? bias[col] : 0.f;
+  float g = 0.f;
+  if constexpr (GATED) g = gate[col];
+  OUT *yc = y + 4 * h * ldy + col;
+#pragma unroll
+  for (int mb = 0; mb < kMB; ++mb)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int64_t ro = mb * 32 + 8 * (e >> 2) + (e & 3);
+      if (4 * h + ro < m) {
+        const float o = act_out<OUT>(acc[mb][e] + bv, la);
+        if constexpr (GATED) yc[ro * ldy] = __builtin_fmaf(g, o, yc[ro * ldy]);
+        else store_out<OUT>(yc + ro * ldy, o);
+      }
+    }
+}
+
 // Tail tiles split over K: y = epi(sum of the kparts raw sums in part order
 // + bias), one thread per 4 columns of a tile row.
 template <typename OUT, int kFM, int kFN>
@@ -565,6 +783,21 @@ static void launch_fast(const WView &w, int64_t n, int64_t k, int64_t ntiles_w, 
                      kp, partial);
 }
 
+template <int FM, int FN>
+static void launch_reduce(const float *partial, int kp, int full, int tiles_n, int tiles_m, int64_t m, int64_t n, void *y,
+                          int y_type, int64_t ldy, const float *bias, const float *gate, int act, hipStream_t stream) {
+  const dim3 rgrid(FM * FN / 4 / 256, (unsigned)(tiles_m * tiles_n - full));
+  const uintptr_t ya = y_type == F32 ? 15 : 7;
+  const int vec = (reinterpret_cast<uintptr_t>(y) & ya) == 0 && ldy % 4 == 0 &&
+                  (reinterpret_cast<uintptr_t>(bias) & 15) == 0 && (reinterpret_cast<uintptr_t>(gate) & 15) == 0;
+  if (y_type == F32)
+    hipLaunchKernelGGL((gemm_tail_reduce_kernel<float, FM, FN>), rgrid, dim3(256), 0, stream, partial, kp, full, tiles_n, m,
+                       n, static_cast<float *>(y), ldy, bias, gate, act, vec);
+  else
+    hipLaunchKernelGGL((gemm_tail_reduce_kernel<__bf16, FM, FN>), rgrid, dim3(256), 0, stream, partial, kp, full, tiles_n,
+                       m, n, static_cast<__bf16 *>(y), ldy, bias, gate, act, vec);
+}
+
 // One weight type's fast GEMM with FM-row block tiles of W waves (W * 32
 // output features), and the reduce of its split tail tiles.
 template <int FM, int W>
@@ -588,24 +821,61 @@ static void launch_fast_fm(const WView &w, int64_t n, int64_t k, int64_t ntiles_
   else
     launch_fast<__bf16, false, FM, W>(w, n, k, ntiles_w, a, m, lda, y, ldy, bias, nullptr, act, tiles_m, tiles_n,
                                       full, kp, partial, wgs, stream);
-  if (split) {
-    const dim3 rgrid(FM * FN / 4 / 256, (unsigned)(grid - full));
-    const uintptr_t ya = y_type == F32 ? 15 : 7;
-    const int vec = (reinterpret_cast<uintptr_t>(y) & ya) == 0 && ldy % 4 == 0 &&
-                    (reinterpret_cast<uintptr_t>(bias) & 15) == 0 && (reinterpret_cast<uintptr_t>(gate) & 15) == 0;
-    if (y_type == F32)
-      hipLaunchKernelGGL((gemm_tail_reduce_kernel<float, FM, FN>), rgrid, dim3(256), 0, stream, partial, kp, full,
-                         tiles_n, m, n, static_cast<float *>(y), ldy, bias, gate, act, vec);
-    else
-      hipLaunchKernelGGL((gemm_tail_reduce_kernel<__bf16, FM, FN>), rgrid, dim3(256), 0, stream, partial, kp, full,
-                         tiles_n, m, n, static_cast<__bf16 *>(y), ldy, bias, gate, act, vec);
+  if (split)
+    launch_reduce<FM, FN>(partial, kp, full, tiles_n, tiles_m, m, n, y, y_type, ldy, bias, gate, act, stream);
+}
+
+template <typename OUT, bool GATED, int FM>
+static void launch_skinny(const WView &w, int64_t n, int64_t k, int64_t ntiles_w, const void *a, int a_type, int64_t m,
+                          int64_t lda, void *y, int64_t ldy, const float *bias, const float *gate, int act, int kp,
+                          float *partial, hipStream_t stream) {
+  const int tiles = (int)((n + 127) / 128);
+  auto go = [&]<typename XT>() {
+    hipLaunchKernelGGL((gemm_skinny_kernel<MQ_GEMM_TYPE, XT, OUT, GATED, FM>), dim3((unsigned)(tiles * kp)), dim3(512), 0,
+                       stream, w, n, k, ntiles_w, static_cast<const XT *>(a), m, lda, static_cast<OUT *>(y), ldy, bias,
+                       gate, act, kp, partial);
+  };
+  if constexpr (skinny_f32(MQ_GEMM_TYPE, FM)) {
+    if (a_type == F32) {
+      go.template operator()<float>();
+      return;
+    }
   }
+  go.template operator()<__bf16>();
+}
+
+// Few rows: FM-row tiles of the whole of x, K in kparts parts.
+template <int FM>
+static void launch_skinny_fm(const WView &w, int64_t n, int64_t k, int64_t ntiles_w, const void *a, int a_type, int64_t m,
+                             int64_t lda, void *y, int y_type, int64_t ldy, const float *bias, const float *gate, int act,
+                             const GemmTail &tail, float *partial, hipStream_t stream) {
+  const int kp = partial ? tail.kparts : 1;
+  if (gate)
+    launch_skinny<float, true, FM>(w, n, k, ntiles_w, a, a_type, m, lda, y, ldy, bias, gate, act, kp, partial, stream);
+  else if (y_type == F32)
+    launch_skinny<float, false, FM>(w, n, k, ntiles_w, a, a_type, m, lda, y, ldy, bias, nullptr, act, kp, partial, stream);
+  else
+    launch_skinny<__bf16, false, FM>(w, n, k, ntiles_w, a, a_type, m, lda, y, ldy, bias, nullptr, act, kp, partial, stream);
+  if (kp > 1)
+    launch_reduce<FM, 128>(partial, kp, 0, (int)((n + 127) / 128), 1, m, n, y, y_type, ldy, bias, gate, act, stream);
 }
 
 template <int T>
-hipError_t launch_gemm_type(const WView &w, int64_t n, int64_t k, int64_t ntiles_w, const __bf16 *a, int64_t m,
+hipError_t launch_gemm_type(const WView &w, int64_t n, int64_t k, int64_t ntiles_w, const void *x, int x_type, int64_t m,
                             int64_t lda, void *y, int y_type, int64_t ldy, const float *bias, const float *gate,
                             int act, const GemmTail &tail, float *partial, hipStream_t stream) {
+  if (tail.skinny) {
+    auto go = [&]<int FM>() {
+      launch_skinny_fm<FM>(w, n, k, ntiles_w, x, x_type, m, lda, y, y_type, ldy, bias, gate, act, tail, partial, stream);
+    };
+    if (x_type != BF16 && !skinny_f32(T, tail.fm)) return hipErrorInvalidValue;
+    if (tail.fm == 32) go.template operator()<32>();
+    else if (tail.fm == 64) go.template operator()<64>();
+    else go.template operator()<96>();
+    return hipGetLastError();
+  }
+  if (x_type != BF16) return hipErrorInvalidValue;  // the other kernels read bf16 x
+  const __bf16 *a = static_cast<const __bf16 *>(x);
   if (gemm_fast_ok(T, m, k, lda)) {
     if (tail.fm == 64)
       launch_fast_fm<64, 4>(w, n, k, ntiles_w, a, m, lda, y, y_type, ldy, bias, gate, act, tail, partial, stream);
@@ -628,7 +898,7 @@ hipError_t launch_gemm_type(const WView &w, int64_t n, int64_t k, int64_t ntiles
   return hipGetLastError();
 }
 
-template hipError_t launch_gemm_type<MQ_GEMM_TYPE>(const WView &, int64_t, int64_t, int64_t, const __bf16 *,
+template hipError_t launch_gemm_type<MQ_GEMM_TYPE>(const WView &, int64_t, int64_t, int64_t, const void *, int,
                                                    int64_t, int64_t, void *, int, int64_t, const float *,
                                                    const float *, int, const GemmTail &, float *, hipStream_t);
 
@@ -706,6 +976,41 @@ int gemm_tile_m(int type, int64_t m, int64_t n, int64_t k, int cus) {
   return best;
 }
 
+// The few-rows kernel (gemm_skinny_kernel): m up to 96, in row tiles of 32, 64
+// or 96, K in whole units, 16-byte aligned rows of f32 or bf16 x.  Above 96
+// rows, and above 32 on a weight of more than 112 128-feature tiles, which
+// fill the chip with whole-K tiles anyway, the 64- and 128-row tiles are as
+// fast or faster (m = 128: 4096 x 4096 Q8_0 19.1 us against 19.7 here; m = 77
+// on 21504 features 33.1 against 33.8); so they are from 65 rows on where a
+// stream does not split K (m = 77, 3072 -> 9216: 30.2 against 32.8).  Below
+// that (us, before / now, bf16 x): 9 x 4096 -> 4096 Q8_0 16.2 / 10.9, 64
+// 16.3 / 14.5, 77 17.3 / 15.7, 77 x 4096 -> 10240 28.5 / 21.8, 32 x 12288 ->
+// 3072 Q2_K 19.1 / 13.2, 77 x 3072 -> 3072 Q4_K 15.6 / 12.2.
+bool gemm_skinny_ok(int type, int64_t m, int64_t n, int64_t k, bool split) {
+  return m <= 96 && (m <= 64 || split) && (m <= 32 || n <= 112 * 128) && k % gemm_unit_k(type) == 0;
+}
+
+// Its plan: a 128-feature tile holds a CU's LDS alone (two fit up to 32 rows),
+// so K is split to about one round of them, at least one chunk of K a part.
+GemmTail gemm_skinny_plan(int64_t m, int64_t n, int64_t k, int cus, bool split) {
+  const int fm = (int)((m + 31) / 32 * 32);
+  const int64_t tiles = (n + 127) / 128, slots = (int64_t)cus * (fm == 32 ? 2 : 1), kc = fm <= 64 ? 512 : 256;
+  int64_t kp = split ? slots / tiles : 1;
+  kp = kp < (k + kc - 1) / kc ? kp : (k + kc - 1) / kc;
+  kp = kp < kGemmMaxKParts ? kp : kGemmMaxKParts;
+  if (kp < 2) return GemmTail{(int)tiles, 1, fm, true};
+  return GemmTail{0, (int)kp, fm, true};
+}
+
+// f32 x read in place, every tile rounding it again, saves the staging pass and
+// loses where many tiles or chunks do so (us, in place / staged: 9 x 4096 ->
+// 4096 11.8 / 13.7, 64 15.5 / 17.0, 77 17.5 / 18.2; 9 x 4096 -> 10240 23.5 / 19.4,
+// 77 x 10240 -> 4096 26.3 / 24.1).
+bool gemm_skinny_reads_f32(int type, int64_t n, int64_t k, const GemmTail &t) {
+  const int64_t kc = t.fm <= 64 ? 512 : 256;
+  return skinny_f32(type, t.fm) && n <= 48 * 128 && (k + kc - 1) / kc <= 2 * t.kparts;
+}
+
 GemmTail gemm_tail_plan(int type, int64_t m, int64_t n, int64_t k, int cus, bool split) {
   const int fm = gemm_tile_m(type, m, n, k, cus);
   const int fn = gemm_tile_n(fm);
@@ -727,13 +1032,13 @@ size_t gemm_tail_bytes(const GemmTail &t, int64_t m, int64_t n) {
   return (size_t)(tiles - t.full_tiles) * t.kparts * t.fm * fn * sizeof(float);
 }
 
-hipError_t launch_gemm(int type, const WView &w, int64_t n, int64_t k, int64_t ntiles_w, const __bf16 *a,
+hipError_t launch_gemm(int type, const WView &w, int64_t n, int64_t k, int64_t ntiles_w, const void *x, int x_type,
                        int64_t m, int64_t lda, void *y, int y_type, int64_t ldy, const float *bias,
                        const float *gate, int act, const GemmTail &tail, float *partial, hipStream_t stream) {
   if (m <= 0 || n <= 0) return hipSuccess;
   hipError_t err = hipErrorInvalidValue;
   dispatch_type(type, [&]<int T>() {
-    err = launch_gemm_type<T>(w, n, k, ntiles_w, a, m, lda, y, y_type, ldy, bias, gate, act, tail, partial, stream);
+    err = launch_gemm_type<T>(w, n, k, ntiles_w, x, x_type, m, lda, y, y_type, ldy, bias, gate, act, tail, partial, stream);
   });
   return err;
 }

@@ -57,8 +57,8 @@ hipError_t launch_gemv(int type, const WView &w, int64_t n, int64_t k, const voi
                        int64_t ldx, void *y, int y_type, int64_t ldy, const float *bias, int act,
                        float *partial, int cus, hipStream_t stream);
 
-// Fused dequant -> bf16 MFMA GEMM.  a is bf16 [m, lda] with lda a multiple
-// of 64 covering ceil(k/64)*64 zero-padded columns.  With `gate` (f32 [n],
+// Fused dequant -> bf16 MFMA GEMM.  x is bf16 [m, lda] with lda a multiple
+// of 64 covering ceil(k/64)*64 zero-padded columns (or f32 with a skinny plan).  With `gate` (f32 [n],
 // f32 y only) the output is the gated residual update
 // y = y + gate * act(a . W^T + bias); without it y = act(a . W^T + bias).
 // The fast kernel (k a whole number of the type's 128- or 256-weight units)
@@ -81,7 +81,8 @@ constexpr int kGemmMaxKParts = 8;
 struct GemmTail {
   int full_tiles;  // tiles run whole (all of them when kparts == 1)
   int kparts;      // K parts per tail tile
-  int fm;          // rows per block tile: 256, or 128 / 64 for small m
+  int fm;          // rows per block tile: 256, or 128 / 64 for small m; 32 .. 96 with skinny
+  bool skinny = false;  // the few-rows kernel, which also reads f32 x
 };
 // K unit of the fast kernel per weight type (the decoder's unit in mq_bfrag.h).
 inline int gemm_unit_k(int type) { return type == Q8_0 ? 128 : 256; }
@@ -95,13 +96,23 @@ size_t gemm_tail_bytes(const GemmTail &t, int64_t m, int64_t n);
 inline bool gemm_fast_ok(int type, int64_t m, int64_t k, int64_t lda) {
   return (k % gemm_unit_k(type)) == 0 && lda % 8 == 0 && (m + kGemmTileM) * lda * 2 < (int64_t(1) << 31);
 }
+// Whether the few-rows kernel takes a call's shape, its plan, and whether it
+// then reads f32 x in place (16-byte aligned rows) rather than staged as bf16.
+bool gemm_skinny_ok(int type, int64_t m, int64_t n, int64_t k, bool split);
+GemmTail gemm_skinny_plan(int64_t m, int64_t n, int64_t k, int cus, bool split);
+bool gemm_skinny_reads_f32(int type, int64_t n, int64_t k, const GemmTail &t);
+// Types whose f32 instance holds its registers: at 96 rows the next chunk's x
+// waits in 48 of them beside two chunks' weights, which spills for the widest.
+constexpr bool skinny_f32(int type, int fm) {
+  return fm <= 64 || !(type == Q5_0 || type == Q5_1 || type == Q5_K || type == Q6_K);
+}
 hipError_t launch_gemm(int type, const WView &w, int64_t n, int64_t k, int64_t ntiles_w,
-                       const __bf16 *a, int64_t m, int64_t lda, void *y, int y_type, int64_t ldy,
+                       const void *x, int x_type, int64_t m, int64_t lda, void *y, int y_type, int64_t ldy,
                        const float *bias, const float *gate, int act, const GemmTail &tail, float *partial,
                        hipStream_t stream);
 // One weight type's launcher (instantiated in its own translation unit).
 template <int T>
-hipError_t launch_gemm_type(const WView &w, int64_t n, int64_t k, int64_t ntiles_w, const __bf16 *a, int64_t m,
+hipError_t launch_gemm_type(const WView &w, int64_t n, int64_t k, int64_t ntiles_w, const void *x, int x_type, int64_t m,
                             int64_t lda, void *y, int y_type, int64_t ldy, const float *bias, const float *gate,
                             int act, const GemmTail &tail, float *partial, hipStream_t stream);
 
