@@ -1011,8 +1011,36 @@ bool gemm_skinny_reads_f32(int type, int64_t n, int64_t k, const GemmTail &t) {
   return skinny_f32(type, t.fm) && n <= 48 * 128 && (k + kc - 1) / kc <= 2 * t.kparts;
 }
 
+// Estimated time (us) of a launch whose tiles of fm rows are one partial round,
+// split into kp parts of K: K steps of 64 at the rate measured for that many
+// workgroups per CU (256-row tiles 1.28 us a step with 96 of the 256 CUs busy to
+// 1.6 with 216; 128-row tiles 0.70 with one workgroup per CU, 1.0 with two,
+// 1.4-1.6 with three; K = 3072 and 4096, Q4_K / Q8_0 / Q2_K), and for a split the
+// reduce launch and the partial sums at 5.3 TB/s.  Within 10 % of 40 measured
+// launches at m = 300 .. 1024.
+static double partial_round_us(int fm, int64_t tiles, int64_t kp, int64_t k, int cus) {
+  const double per_cu = (double)(tiles * kp) / cus, steps = (double)k / 64 / kp;
+  const double step = fm == 256 ? 0.98 + 0.8 * (per_cu < 1 ? per_cu : 1) : per_cu <= 1 ? 0.70 : per_cu <= 2 ? 1.0 : 1.6;
+  const double sums = kp < 2 ? 0.0 : 5.0 + (double)(tiles * kp) * fm * gemm_tile_n(fm) * 4 / 5.3e6;
+  return steps * step + sums;
+}
+
 GemmTail gemm_tail_plan(int type, int64_t m, int64_t n, int64_t k, int cus, bool split) {
-  const int fm = gemm_tile_m(type, m, n, k, cus);
+  int fm = gemm_tile_m(type, m, n, k, cus);
+  if (split && fm == 256) {
+    // Less than one round of 256-row tiles: 128-row tiles, split by their own
+    // rule, where they are estimated clearly cheaper: fewer padded rows (300 x
+    // 3072 -> 9216 Q4_K 41.8 -> 35.7 us, 300 x 5120 -> 5120 Q6_K 41.4 -> 34.4) or
+    // no partial sums at a good fill (512 x 3072 -> 12288 52.7 -> 48.3).
+    const int64_t t256 = ((m + 255) / 256) * ((n + 255) / 256), t128 = ((m + 127) / 128) * ((n + 127) / 128);
+    if (t256 < cus) {
+      int64_t rem = 0;
+      const int64_t kp256 = tail_kparts(type, m, n, k, cus, 256, &rem, false);
+      const int64_t kp128 = tail_kparts(type, m, n, k, cus, 128, &rem, false);
+      if (rem == t128 && partial_round_us(128, t128, kp128, k, cus) < 0.92 * partial_round_us(256, t256, kp256, k, cus))
+        fm = 128;
+    }
+  }
   const int fn = gemm_tile_n(fm);
   const int64_t tiles = ((m + fm - 1) / fm) * ((n + fn - 1) / fn);
   GemmTail t{(int)tiles, 1, fm};
