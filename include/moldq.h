@@ -360,6 +360,25 @@ int mq_gguf_version(const mq_gguf *g);
 int mq_lora_apply(float *w, int64_t ldw, int64_t rows, int64_t k, const float *b, int64_t ldb,
                   const float *a, int64_t lda, int rank, float scale, void *stream);
 
+/* The whole merge of one k-quant weight (Q2_K .. Q6_K) in one pass: decoded to
+ * f32, each patch applied on its rows in order as mq_lora_apply does, and
+ * quantized back to its type into a new tensor.  The blocks equal those of
+ * mq_dequantize, mq_lora_apply per patch and mq_quantize.  At most
+ * MQ_LORA_MAX_PATCHES patches, their rows inside the weight (MQ_E_UNSUPPORTED
+ * for more, or another type: the separate calls serve them).  Runs on `stream`
+ * and returns when the blocks are in place. */
+#define MQ_LORA_MAX_PATCHES 8
+typedef struct mq_lora_patch {
+    const float *b;     /* device f32 [rows, ldb] */
+    const float *a;     /* device f32 [rank, lda], k columns */
+    int64_t ldb, lda;
+    int64_t row0, rows; /* target rows of the weight */
+    int32_t rank;
+    float scale;
+} mq_lora_patch;
+int mq_lora_merge(mq_ctx *ctx, const mq_qtensor *w, const mq_lora_patch *patches, int count, void *stream,
+                  mq_qtensor **out);
+
 /* --- GGUF metadata (candle gguf_file::Content::metadata).  Value types are
  *     GGUF's: 0 u8, 1 i8, 2 u16, 3 i16, 4 u32, 5 i32, 6 f32, 7 bool,
  *     8 string, 9 array, 10 u64, 11 i64, 12 f64.  An array reports type 9,

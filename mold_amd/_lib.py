@@ -17,6 +17,14 @@ MQ_X_Q8K, MQ_X_Q8K_BLOCK_BYTES = 100, 304   # mq_quantize_x_q8k's activation blo
 # Every symbol include/moldq.h declares, with (restype, argtypes).
 _vp, _i64, _int, _sz = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_size_t
 _pp = ctypes.POINTER(ctypes.c_void_p)
+class LoraPatchC(ctypes.Structure):
+    """mq_lora_patch"""
+    _fields_ = [("b", ctypes.c_void_p), ("a", ctypes.c_void_p), ("ldb", ctypes.c_int64), ("lda", ctypes.c_int64),
+                ("row0", ctypes.c_int64), ("rows", ctypes.c_int64), ("rank", ctypes.c_int32), ("scale", ctypes.c_float)]
+
+
+MQ_LORA_MAX_PATCHES = 8
+
 SIGNATURES = {
     "mq_last_error": (ctypes.c_char_p, []),
     "mq_version": (_int, []),
@@ -33,6 +41,7 @@ SIGNATURES = {
     "mq_qtensor_from_device": (_int, [_vp, _int, _i64, _i64, _vp, _sz, _vp, _pp]),
     "mq_quantize": (_int, [_vp, _int, _i64, _i64, _vp, _i64, _vp, _pp]),
     "mq_lora_apply": (_int, [_vp, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _int, ctypes.c_float, _vp]),
+    "mq_lora_merge": (_int, [_vp, _vp, ctypes.POINTER(LoraPatchC), _int, _vp, _pp]),
     "mq_quantize_fp8": (_int, [_vp, _int, _i64, _i64, _vp, _i64, ctypes.c_float, _vp, _pp]),
     "mq_qtensor_download": (_int, [_vp, _vp, _vp, _sz]),
     "mq_qtensor_concat_rows": (_int, [_vp, _vp, _i64, _pp]),

@@ -717,6 +717,39 @@ int mq_quantize_fp8(mq_ctx *ctx, int dtype, int64_t n, int64_t k, const void *sr
   return quantize_common(ctx, "mq_quantize_fp8", dtype, n, k, src, true, ld, scale, stream, out);
 }
 
+int mq_lora_merge(mq_ctx *ctx, const mq_qtensor *w, const mq_lora_patch *patches, int count, void *stream,
+                  mq_qtensor **out) {
+  if (!ctx || !w || !out || (!patches && count > 0)) return fail(MQ_E_INVALID, "mq_lora_merge: NULL argument");
+  *out = nullptr;
+  if (count < 0) return fail(MQ_E_INVALID, "mq_lora_merge: count=%d < 0", count);
+  if (!is_quant(w->dtype) || type_info(w->dtype).bs != 256)
+    return fail(MQ_E_UNSUPPORTED, "mq_lora_merge: weight type %d is not a k-quant", w->dtype);
+  if (count > MQ_LORA_MAX_PATCHES)
+    return fail(MQ_E_UNSUPPORTED, "mq_lora_merge: %d patches, at most %d", count, MQ_LORA_MAX_PATCHES);
+  LoraPatches lp{};
+  lp.count = count;
+  for (int i = 0; i < count; ++i) {
+    const mq_lora_patch &q = patches[i];
+    if (!q.a || !q.b) return fail(MQ_E_INVALID, "mq_lora_merge: patch %d: NULL pointer", i);
+    if (q.rank < 1 || q.ldb < q.rank || q.lda < w->k || q.row0 < 0 || q.rows < 0 || q.row0 > w->n - q.rows)
+      return fail(MQ_E_INVALID, "mq_lora_merge: patch %d: bad rank, leading dimension or rows", i);
+    lp.p[i] = LoraPatch{q.b, q.a, q.ldb, q.lda, q.row0, q.rows, q.rank, q.scale};
+  }
+  DeviceGuard g(ctx->device);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  mq_qtensor *t = nullptr;
+  const int rc = make_tensor(ctx, w->dtype, w->n, w->k, &t);
+  if (rc) return rc;
+  hipError_t e = launch_lora_merge(w->dtype, view_of(w), t->geo, lp, t->data, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  if (e != hipSuccess) {
+    mq_qtensor_free(t);
+    return hip_fail(e, "LoRA merge");
+  }
+  *out = t;
+  return MQ_OK;
+}
+
 int mq_qtensor_download(mq_ctx *ctx, const mq_qtensor *w, void *host_blocks, size_t nbytes) {
   if (!ctx || !w || !host_blocks) return fail(MQ_E_INVALID, "mq_qtensor_download: NULL argument");
   if (nbytes != w->gguf_bytes) return fail(MQ_E_INVALID, "download needs %zu bytes, got %zu", w->gguf_bytes, nbytes);

@@ -18,6 +18,19 @@ hipError_t launch_repack(int type, const void *src, void *dst, const Geo &g, boo
 // included.
 hipError_t launch_quantize(int type, const void *src, bool fp8, int64_t ld, float scale, void *tiled, const Geo &g,
                            hipStream_t stream);
+// Patches of a one-pass LoRA merge of a k-quant weight (mq_lora_merge).
+struct LoraPatch {
+  const float *b, *a;   // [rows, ldb], [rank, lda]
+  int64_t ldb, lda, row0, rows;
+  int rank;
+  float scale;
+};
+struct LoraPatches {
+  int count;
+  LoraPatch p[MQ_LORA_MAX_PATCHES];
+};
+hipError_t launch_lora_merge(int type, const WView &w, const Geo &g, const LoraPatches &patches, void *tiled,
+                             hipStream_t stream);
 hipError_t launch_dequant(int type, const WView &w, int64_t n, int64_t k, void *dst, int dst_type,
                           hipStream_t stream);
 // Dense GGUF tensors (F32 / F16 / BF16): src[n, lds] of src_type -> dst[n,

@@ -763,6 +763,86 @@ __global__ __launch_bounds__(256) void quantize_k_kernel(const void *__restrict_
   quantize_sub<TYPE, N>(x, real, j, tiled, g, (row / kRowTile) * g.nb + b, (int)(row % kRowTile));
 }
 
+// A LoRA merge in one pass: the weight's own values (decoded as dequantize
+// does), plus each patch's (b . a) * scale on its rows, quantized again; the
+// steps and their order are those of dequantize, lora_apply per patch and
+// quantize, so the blocks are the same.  Bound by the search's VALU work as
+// quantize_k_kernel is: the rank's fmas add 32 operations a value at rank 32 to
+// about 430, where the three passes moved 28 bytes a value through HBM (Q4_K
+// [21504, 3072], four rank-32 patches: 55 + 234 + 640 us, in one pass 700; the
+// merge call 1003 -> 728).  A patch's a
+// (kLoraR ranks of the workgroup's 256 columns) and b are staged in LDS, a
+// with the lanes' 16-byte pieces side by side (piece c of sub-block j at
+// c * lanes + j: the lanes of a row read 128 or 256 consecutive bytes).
+constexpr int kLoraR = 32;
+
+template <int TYPE>
+__global__ __launch_bounds__(256, 2) void lora_merge_kernel(WView w, Geo g, LoraPatches patches, uint8_t *__restrict__ tiled) {
+  constexpr int kL = kq_lanes<TYPE>(), N = 256 / kL, kRows = 256 / kL;
+  __shared__ __align__(16) float as[kLoraR][256];
+  __shared__ float bs[kLoraR][kRows];
+  const int tid = threadIdx.x, j = tid % kL, rl = tid / kL;
+  const int64_t rg = blockIdx.x / (uint32_t)g.nb, blk = blockIdx.x - rg * g.nb;
+  const int64_t row0 = rg * kRows, row = row0 + rl;
+  const bool real = row < g.n;
+  const int64_t tile = row / kRowTile;
+  const int r64 = (int)(row % kRowTile);
+  float x[N];
+#pragma unroll
+  for (int c = 0; c < N / 8; ++c) {
+    float v[8];
+    decode8<TYPE>(w, tile, r64, blk, j * N + 8 * c, v);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      // the f32 weight itself: without this the decoder's last multiply-add may
+      // move past the patch's add
+      asm volatile("" : "+v"(v[i]));
+      x[8 * c + i] = v[i];
+    }
+  }
+  for (int p = 0; p < patches.count; ++p) {
+    const LoraPatch &q = patches.p[p];
+    if (row0 + kRows <= q.row0 || row0 >= q.row0 + q.rows) continue;  // none of the workgroup's rows
+    const bool mine = row >= q.row0 && row < q.row0 + q.rows;
+    float d[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) d[i] = 0.f;
+    for (int r0 = 0; r0 < q.rank; r0 += kLoraR) {
+      const int rn = q.rank - r0 < kLoraR ? q.rank - r0 : kLoraR;
+      __syncthreads();  // the chunk before is read
+      for (int e = tid; e < rn * 256; e += 256) {
+        const int rr = e >> 8, col = e & 255, sub = col / N, in = col % N;
+        as[rr][((in >> 2) * kL + sub) * 4 + (in & 3)] = q.a[(int64_t)(r0 + rr) * q.lda + blk * 256 + col];
+      }
+      for (int e = tid; e < rn * kRows; e += 256) {
+        const int rr = e / kRows, ii = e % kRows;
+        const int64_t pr = row0 + ii - q.row0;
+        bs[rr][ii] = pr >= 0 && pr < q.rows ? q.b[pr * q.ldb + r0 + rr] : 0.f;
+      }
+      __syncthreads();
+      for (int rr = 0; rr < rn; ++rr) {
+        const float bv = bs[rr][rl];
+#pragma unroll
+        for (int c = 0; c < N / 4; ++c) {
+          const float4 av = *reinterpret_cast<const float4 *>(&as[rr][(c * kL + j) * 4]);
+          d[4 * c] = __builtin_fmaf(bv, av.x, d[4 * c]);
+          d[4 * c + 1] = __builtin_fmaf(bv, av.y, d[4 * c + 1]);
+          d[4 * c + 2] = __builtin_fmaf(bv, av.z, d[4 * c + 2]);
+          d[4 * c + 3] = __builtin_fmaf(bv, av.w, d[4 * c + 3]);
+        }
+      }
+    }
+    if (mine) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const float t = d[i] * q.scale;
+        x[i] = x[i] + t;
+      }
+    }
+  }
+  quantize_sub<TYPE, N>(x, real, j, tiled, g, tile * g.nb + blk, r64);
+}
+
 template <bool FP8>
 hipError_t launch_quantize_src(int type, const void *src, int64_t ld, float scale, void *tiled, const Geo &g,
                                      hipStream_t stream) {
@@ -793,6 +873,21 @@ hipError_t launch_quantize_src(int type, const void *src, int64_t ld, float scal
 }
 
 }  // namespace
+
+hipError_t launch_lora_merge(int type, const WView &w, const Geo &g, const LoraPatches &patches, void *tiled,
+                             hipStream_t stream) {
+  if (g.n == 0 || g.nb == 0) return hipSuccess;
+  bool ok = false;
+  dispatch_type(type, [&]<int T>() {
+    if constexpr (type_info(T).bs == 256) {
+      const dim3 grid((unsigned)(g.nb * (g.ntiles * kRowTile * kq_lanes<T>() / 256)));
+      hipLaunchKernelGGL((lora_merge_kernel<T>), grid, dim3(256), 0, stream, w, g, patches, static_cast<uint8_t *>(tiled));
+      ok = true;
+    }
+  });
+  if (!ok) return hipErrorInvalidValue;
+  return hipGetLastError();
+}
 
 hipError_t launch_quantize(int type, const void *src, bool fp8, int64_t ld, float scale, void *tiled, const Geo &g,
                            hipStream_t stream) {

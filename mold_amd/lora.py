@@ -154,39 +154,59 @@ def build_patches(adapter: LoraAdapter, scale: float) -> Tuple[Dict[str, List[Lo
     return patches, skipped
 
 
+def _device_factors(b, a, device, rows: int, k: int):
+    """A patch's factors as contiguous f32 on the weight's device, shapes checked."""
+    import torch
+    b = b.to(device=device, dtype=torch.float32).contiguous()
+    a = a.to(device=device, dtype=torch.float32).contiguous()
+    rank = a.shape[0]
+    if b.shape != (rows, rank) or a.shape != (rank, k):
+        raise ValueError(f"LoRA shapes b {tuple(b.shape)} a {tuple(a.shape)} do not fit rows {rows} x k {k}")
+    return b, a
+
+
 def lora_apply(w, b, a, scale: float, stream=None) -> None:
     """w[rows, k] += (b . a) * scale in place on device f32 tensors (mq_lora_apply)."""
     import torch
     assert w.dtype == torch.float32 and w.dim() == 2 and w.stride(1) == 1
-    b = b.to(device=w.device, dtype=torch.float32).contiguous()
-    a = a.to(device=w.device, dtype=torch.float32).contiguous()
     rows, k = w.shape
+    b, a = _device_factors(b, a, w.device, rows, k)
     rank = a.shape[0]
-    if b.shape != (rows, rank) or a.shape != (rank, k):
-        raise ValueError(f"LoRA shapes b {tuple(b.shape)} a {tuple(a.shape)} do not fit rows {rows} x k {k}")
     check(_lib.load().mq_lora_apply(w.data_ptr(), w.stride(0), rows, k, b.data_ptr(), rank, a.data_ptr(), k, rank,
                                     ctypes.c_float(scale), _stream_ptr(stream)))
 
 
-def patch_qtensor(qt: QTensor, patches: List[LoraPatch]) -> Tuple[QTensor, int]:
-    """One targeted tensor (lora.rs:748-849) on the device: dequantize to f32,
-    apply each patch (whole tensor, or its fused row slice; an out-of-range
-    slice is skipped as mold does), re-quantize to the original type.
-    Returns (new tensor, patches applied)."""
-    t = qt.dequantize()
-    base_rows = t.shape[0]
-    applied = 0
+def _targets(patches: List[LoraPatch], base_rows: int):
+    """(patch, first row, rows) of the patches that apply: the whole tensor or a fused row
+    slice (an out-of-range slice is skipped as mold does)."""
     for p in patches:
+        off, size = 0, base_rows
         if p.target.fused:
             off, size = fused_slice_range(base_rows, p.b.shape[0], p.target.component, p.target.num_components)
             if off + size > base_rows:
                 continue
-            lora_apply(t[off:off + size], p.b, p.a, p.effective_scale)
-        else:
-            lora_apply(t, p.b, p.a, p.effective_scale)
-        applied += 1
-    out = QTensor.quantize(qt.device, t, qt.dtype())
-    return out, applied
+        yield p, off, size
+
+
+def patch_qtensor(qt: QTensor, patches: List[LoraPatch]) -> Tuple[QTensor, int]:
+    """One targeted tensor (lora.rs:748-849) on the device: dequantize to f32,
+    apply each patch, re-quantize to the original type; a k-quant in one pass
+    (mq_lora_merge: the same blocks).  Returns (new tensor, patches applied)."""
+    n, k = qt.shape
+    todo = list(_targets(patches, n))
+    if qt.dtype().block_size() == 256 and 1 <= len(todo) <= _lib.MQ_LORA_MAX_PATCHES \
+            and all(off >= 0 and size >= 0 and p.a.shape[0] >= 1 for p, off, size in todo):
+        keep = [_device_factors(p.b, p.a, f"cuda:{qt.device.ordinal}", size, k) for p, _, size in todo]
+        arr = (_lib.LoraPatchC * len(todo))(*[
+            _lib.LoraPatchC(b.data_ptr(), a.data_ptr(), a.shape[0], k, off, size, a.shape[0], p.effective_scale)
+            for (p, off, size), (b, a) in zip(todo, keep)])
+        h = ctypes.c_void_p()
+        check(_lib.load().mq_lora_merge(qt.device.handle, qt.handle, arr, len(todo), _stream_ptr(), ctypes.byref(h)))
+        return QTensor(qt.device, h), len(todo)
+    t = qt.dequantize()
+    for p, off, size in todo:
+        lora_apply(t[off:off + size], p.b, p.a, p.effective_scale)
+    return QTensor.quantize(qt.device, t, qt.dtype()), len(todo)
 
 
 def gguf_lora_var_builder(transformer_path: str, adapter: LoraAdapter, scale: float, device: Device):
