@@ -289,7 +289,11 @@ int mq_attn_pad_correct(const void *o, int64_t batch, int heads, int64_t rows, i
  * Asynchronous on stream. */
 int mq_attention_bf16(const void *q, const void *k, const void *v, int64_t batch, int heads, int64_t l_total,
                       int head_dim, int64_t valid, const int64_t *drop, void *out, int64_t out_batch_stride,
-                      int64_t ldo, float *lse, float *guard, void *stream);
+                      int64_t ldo, float *lse, float *guard, void *scratch, size_t scratch_bytes, void *stream);
+/* Device scratch (16-byte aligned, used by that call alone) with which the
+ * call above fills the chip when its query tiles leave a partial round; 0 if
+ * it needs none.  With less, or NULL, it runs without. */
+size_t mq_attention_scratch_size(int64_t batch, int heads, int64_t valid);
 
 /* Quantize activations once for several Q4_K GEMVs: x [m, k] (F32 or BF16,
  * row stride ldx, 16-byte aligned rows) -> m * k / 256 blocks of

@@ -61,7 +61,8 @@ SIGNATURES = {
     "mq_attn_pad_correct": (_int, [_vp, _i64, _int, _i64, _i64, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _i64, _i64,
                                    _vp, _vp]),
     "mq_attention_bf16": (_int, [_vp, _vp, _vp, _i64, _int, _i64, _int, _i64, ctypes.POINTER(_i64), _vp, _i64, _i64, _vp,
-                                 _vp, _vp]),
+                                 _vp, _vp, _sz, _vp]),
+    "mq_attention_scratch_size": (_sz, [_i64, _int, _i64]),
     "mq_gguf_open": (_int, [ctypes.c_char_p, _pp]),
     "mq_gguf_close": (None, [_vp]),
     "mq_gguf_tensor_count": (_i64, [_vp]),

@@ -56,6 +56,8 @@ constexpr int kHd = 128;       // head dim
 constexpr int kKeys = 64;      // keys per block
 constexpr int kMaxBatch = 8;   // elements per launch (their masks are kernel arguments)
 constexpr int kCus = 256;      // MI355X
+constexpr int kMaxParts = 8;   // key shares of a split tile
+constexpr int64_t kPart = 256 * (kHd + 2);  // floats of one share's sums
 
 // Per batch element: kept keys, the masked range's start and length, and the
 // zero keys that the caller's guard counts.
@@ -96,27 +98,59 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
   return u;
 }
 
+// The log-sum-exp and guard of a row with sum l relative to 2^ms, which all
+// lanes of a half wave (or both halves) share or hold one each; `one`: the
+// lane that stores it.  Z + npad, the sum of exp over the kept keys and npad
+// zero scores, is taken relative to 2^max(ms, 0).  Every lane of the wave joins.
+__device__ __forceinline__ void row_sums(float ms, float l, float npad, bool stored, bool one, float *lse,
+                                         unsigned int *guard) {
+  const float top = __builtin_fmaxf(ms, 0.f);
+  const float zero = npad * __builtin_amdgcn_exp2f(-top);
+  const float z = l * __builtin_amdgcn_exp2f(ms - top) + zero;
+  if (lse && stored && one) *lse = 0.69314718055994531f * (top + __builtin_amdgcn_logf(z));
+  if (guard) {
+    float share = stored ? zero / z : 0.f;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+      const float u = __shfl_xor(share, off);
+      share = (u > share || u != u) ? u : share;
+    }
+    const unsigned int bits = __float_as_uint(share);
+    if ((threadIdx.x & 63) == 0 && bits > __hip_atomic_load(guard, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(guard, bits);
+  }
+}
+
 template <int S>
 struct Slot {
   static constexpr int v = S;
 };
 
-template <int W>
+template <int W, bool kSplit>
 __global__ __launch_bounds__(64 * W, 2) void attention_kernel(
     const __bf16 *__restrict__ q, const __bf16 *__restrict__ k, const __bf16 *__restrict__ v, int heads,
     int64_t l_total, int rows, int qtiles, AttnKeys keys, float scale, __bf16 *__restrict__ out, int64_t sb_out,
-    int64_t ldo, float *__restrict__ lse, unsigned int *__restrict__ guard) {
+    int64_t ldo, float *__restrict__ lse, unsigned int *__restrict__ guard, int full_tiles, int kparts,
+    float *__restrict__ partial) {
   __shared__ uint4 lds_k[2][kKeys * kHd / 8];
   __shared__ uint4 lds_v[3][kKeys * kHd / 8];
 
-  // workgroup i runs on XCD i % 8: each XCD takes a contiguous run of
-  // (head, query tile), so one head's K and V stay in its L2
-  const int total = gridDim.x, xcd = blockIdx.x & 7, base = total >> 3, extra = total & 7;
-  const int tile = xcd * base + (xcd < extra ? xcd : extra) + (int)(blockIdx.x >> 3);
+  // Workgroup i runs on XCD i % 8: each XCD takes a contiguous run of (head,
+  // query tile), so one head's K and V stay in its L2.  Tiles from full_tiles
+  // (then a multiple of kCus) on run as kparts workgroups, each over a share of
+  // the keys, whose sums combine_kernel adds.
+  const bool split = kSplit && (int)blockIdx.x >= full_tiles;
+  const int i0 = split ? blockIdx.x - full_tiles : blockIdx.x;
+  const int total = !kSplit ? gridDim.x : split ? gridDim.x - full_tiles : full_tiles;
+  const int xcd = i0 & 7, base = total >> 3, extra = total & 7;
+  const int unit = xcd * base + (xcd < extra ? xcd : extra) + (i0 >> 3);
+  const int tile = split ? full_tiles + unit / kparts : unit, part = split ? unit % kparts : 0;
   const int bh = tile / qtiles, qt = tile - bh * qtiles;
   const int b = bh / heads, head = bh - b * heads;
   const int nk = keys.nk[b], lo = keys.lo[b], gap = keys.gap[b];
-  const int nblk = (nk + kKeys - 1) / kKeys;
+  const int all = (nk + kKeys - 1) / kKeys;
+  const int b0 = split ? part * all / kparts : 0;  // first block of keys
+  const int nblk = (split ? (part + 1) * all / kparts : all) - b0;
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -142,7 +176,7 @@ __global__ __launch_bounds__(64 * W, 2) void attention_kernel(
   auto dma = [&](int blk, int kslot, int vslot) {
 #pragma unroll
     for (int j = 0; j < 16 / W; ++j) {
-      int r = blk * kKeys + drow + 4 * W * j;
+      int r = (b0 + blk) * kKeys + drow + 4 * W * j;
       r = r < nk ? r : nk - 1;
       const uint32_t off = (uint32_t)(r + (r >= lo ? gap : 0)) * (2 * kHd);
       dma16(kbase, off + kch, __builtin_amdgcn_readfirstlane(lkw + kslot * 16384 + 1024 * W * j));
@@ -155,7 +189,9 @@ __global__ __launch_bounds__(64 * W, 2) void attention_kernel(
   for (int d = 0; d < 4; ++d)
 #pragma unroll
     for (int e = 0; e < 16; ++e) o[d][e] = 0.f;
-  float m = -__builtin_inff(), l = 0.f;  // running maximum (both halves) and this half's sum
+  // running maximum (both halves), finite so that scores of -inf before the first
+  // finite one give 0 and not NaN, and this half's sum
+  float m = -__FLT_MAX__, l = 0.f;
 
   const int i16 = lane & 15;
   lds_char *ka[8], *va[4];
@@ -240,6 +276,21 @@ __global__ __launch_bounds__(64 * W, 2) void attention_kernel(
       }
   };
 
+  // a share without keys (masked ranges leave an element fewer blocks than the
+  // plan counted): the whole workgroup returns before its first barrier
+  float *po = nullptr;
+  if constexpr (kSplit)
+    if (split) {
+      po = partial + (int64_t)unit * kPart + (32 * wave + l32) * (int64_t)kHd;
+      if (nblk == 0) {
+        for (int d = 0; d < 16; ++d) *reinterpret_cast<float4 *>(po + 64 * h + 4 * d) = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (h == 0)
+          *reinterpret_cast<float2 *>(partial + (int64_t)unit * kPart + 256 * kHd + 2 * (32 * wave + l32)) =
+              make_float2(-__builtin_inff(), 0.f);
+        return;
+      }
+    }
+
   dma(0, 0, 0);
   block_barrier();
   if (nblk > 1) dma(1, 1, 1);
@@ -252,12 +303,12 @@ __global__ __launch_bounds__(64 * W, 2) void attention_kernel(
   auto block = [&](int i, auto kslot, bool last, bool more) {
     constexpr int ks = decltype(kslot)::v;
     bf16x8 p[2];
-    if (last) mask(s0, i * kKeys);
+    if (last) mask(s0, (b0 + i) * kKeys);
     raise_max(max16(s0));
     scores(ks, 1, s1);
     probs(s0, p);
     accumulate(vs, 0, p);
-    if (last) mask(s1, i * kKeys + 32);
+    if (last) mask(s1, (b0 + i) * kKeys + 32);
     const float mx = max16(s1);
     if (!last) {
       block_barrier();
@@ -286,8 +337,22 @@ __global__ __launch_bounds__(64 * W, 2) void attention_kernel(
   }
 
   l = half_add(l);
-  const float inv = 1.f / l;
   const bool stored = row < rows;
+  if constexpr (kSplit)
+    if (split) {
+      // this share's unscaled O (row-major [256][128]), then (scale m, l) of its rows
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<float4 *>(po + 32 * d + 8 * g + 4 * h) =
+              make_float4(o[d][4 * g], o[d][4 * g + 1], o[d][4 * g + 2], o[d][4 * g + 3]);
+      if (h == 0)
+        *reinterpret_cast<float2 *>(partial + (int64_t)unit * kPart + 256 * kHd + 2 * (32 * wave + l32)) =
+            make_float2(m * scale, l);
+      return;
+    }
+  const float inv = 1.f / l;
   __bf16 *orow = out + (int64_t)b * sb_out + (int64_t)row * ldo + (int64_t)head * kHd;
 #pragma unroll
   for (int d = 0; d < 4; ++d)
@@ -303,39 +368,101 @@ __global__ __launch_bounds__(64 * W, 2) void attention_kernel(
       const auto y = __builtin_amdgcn_permlane32_swap(a1, c1, false, false);
       if (stored) *reinterpret_cast<uint4 *>(orow + 32 * d + 16 * g + 8 * h) = make_uint4(x[0], y[0], x[1], y[1]);
     }
-  if (lse || guard) {
-    // Z + npad relative to 2^top: the sum of exp over the kept keys and npad zero keys
-    const float ms = m * scale, top = __builtin_fmaxf(ms, 0.f);
-    const float zero = keys.npad[b] * __builtin_amdgcn_exp2f(-top);
-    const float z = l * __builtin_amdgcn_exp2f(ms - top) + zero;
-    if (lse && stored && h == 0)
-      lse[(int64_t)bh * rows + row] = 0.69314718055994531f * (top + __builtin_amdgcn_logf(z));
-    if (guard) {
-      float share = stored ? zero / z : 0.f;
-#pragma unroll
-      for (int off = 16; off >= 1; off >>= 1) {
-        const float u = __shfl_xor(share, off);
-        share = (u > share || u != u) ? u : share;
-      }
-      const unsigned int bits = __float_as_uint(share);
-      if (lane == 0 && bits > __hip_atomic_load(guard, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        atomicMax(guard, bits);
-    }
-  }
+  if (lse || guard)
+    row_sums(m * scale, l, keys.npad[b], stored, h == 0, lse ? lse + (int64_t)bh * rows + row : nullptr, guard);
 }
 
-// Waves per workgroup: 8 (256 query rows, one workgroup per CU) or 4 (128
-// rows, two per CU, each with its own K and V tiles).  In units of the 8-wave
-// tile's time a round of 4-wave tiles takes 1.10 with two per CU and 0.76 with
-// one (24 heads x 1100 tokens, 216 of them: 24.8 us against 32.5; 32 x 1100,
-// 288: 36.2 against 32.6), so the variant with the cheaper sum of rounds runs:
-// 4 waves below about 128 8-wave tiles (2 x 4608 tokens 71 us against 99) and
-// where they leave a nearly empty last round (24 x 3500: 161 against 183).
-bool eight_waves(int64_t heads, int64_t rows) {
-  const int64_t t8 = heads * ((rows + 255) / 256), t4 = heads * ((rows + 127) / 128);
-  const int64_t full = t4 / (2 * kCus), rest = t4 % (2 * kCus);
-  const double four = 1.10 * full + (rest == 0 ? 0.0 : rest <= kCus ? 0.76 : 1.10);
-  return (double)((t8 + kCus - 1) / kCus) <= four;
+// The split tiles: a row's parts, each relative to its own maximum, added in
+// part order.  Half a wave per row, 4 columns a lane, every part's load in
+// flight at once: bound by reading the sums (133 KB a share).
+__global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ partial, int kparts, int full_tiles,
+                                                      int heads, int rows, int qtiles, AttnKeys keys,
+                                                      __bf16 *__restrict__ out, int64_t sb_out, int64_t ldo,
+                                                      float *__restrict__ lse, unsigned int *__restrict__ guard) {
+  const int t = blockIdx.y, tile = full_tiles + t;
+  const int bh = tile / qtiles, qt = tile - bh * qtiles;
+  const int b = bh / heads, head = bh - b * heads;
+  const int rl = blockIdx.x * 8 + (threadIdx.x >> 5), l32 = threadIdx.x & 31;
+  const int row = 256 * qt + rl;
+  const float *p0 = partial + (int64_t)t * kparts * kPart;
+  float ms[kMaxParts], ls[kMaxParts];
+  float4 v[kMaxParts];
+  float top = -__builtin_inff();
+#pragma unroll
+  for (int p = 0; p < kMaxParts; ++p)
+    if (p < kparts) {
+      const float2 ml = *reinterpret_cast<const float2 *>(p0 + p * kPart + 256 * kHd + 2 * rl);
+      v[p] = *reinterpret_cast<const float4 *>(p0 + p * kPart + rl * kHd + 4 * l32);
+      ms[p] = ml.x;
+      ls[p] = ml.y;
+      top = __builtin_fmaxf(top, ml.x);
+    }
+  float z = 0.f;
+  float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int p = 0; p < kMaxParts; ++p)
+    if (p < kparts) {
+      const float f = ms[p] == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(ms[p] - top);
+      z = __builtin_fmaf(f, ls[p], z);
+      o.x = __builtin_fmaf(f, v[p].x, o.x);
+      o.y = __builtin_fmaf(f, v[p].y, o.y);
+      o.z = __builtin_fmaf(f, v[p].z, o.z);
+      o.w = __builtin_fmaf(f, v[p].w, o.w);
+    }
+  const float inv = 1.f / z;
+  const bool stored = row < rows;
+  if (stored)
+    *reinterpret_cast<uint2 *>(out + (int64_t)b * sb_out + (int64_t)row * ldo + (int64_t)head * kHd + 4 * l32) =
+        make_uint2(pack2(o.x * inv, o.y * inv), pack2(o.z * inv, o.w * inv));
+  if (lse || guard)
+    row_sums(top, z, keys.npad[b], stored, l32 == 0, lse ? lse + (int64_t)bh * rows + row : nullptr, guard);
+}
+
+// How a launch of `heads` heads x `rows` rows over `keys` keys runs: waves per
+// workgroup, the tiles run whole, and the key shares of the rest.  8 waves: 256
+// query rows, one workgroup per CU.  4 waves: 128 rows, two per CU, each with
+// its own K and V tiles.  The last, partial round of 8-wave tiles may be split
+// over the keys so that it fills the CUs, at the price of the shares' f32 sums
+// (written and read once) and a launch.  The estimates are in us: an 8-wave tile
+// takes 1.85 per block of 64 keys, a round of 4-wave tiles 1.10 of that with
+// two per CU and 0.70 with one (24 heads x 1100 tokens, 216 of them: 24.8 us
+// against 32.5 with 8 waves; 32 x 1100, 288: 36.2 against 32.6; 8 x 3500, 224:
+// 66), sums move at 5 TB/s.  A split has to look 10 % better, since a round that
+// leaves CUs idle clocks higher: measured, whole -> split, heads x tokens: 2 x
+// 4608 82 -> 41 us, 24 x 2816 140 -> 117, 40 x 1664 88 -> 80, 48 x 7145 1279 ->
+// 1181, 24 x 16896 3411 -> 3145; below the line 24 x 7145 620 -> 619, 8 x 3500
+// 66 -> 70, 48 x 4608 558 -> 531.
+struct AttnPlan {
+  int waves, full, kparts;
+};
+AttnPlan attn_plan(int64_t heads, int64_t rows, int64_t keys, bool may_split) {
+  const int64_t t8 = heads * ((rows + 255) / 256), t4 = heads * ((rows + 127) / 128), blocks = (keys + kKeys - 1) / kKeys;
+  const double tile = 1.85 * blocks;
+  const int64_t full4 = t4 / (2 * kCus), rest4 = t4 % (2 * kCus);
+  AttnPlan best{4, (int)t4, 1};
+  double us = tile * (1.10 * full4 + (rest4 == 0 ? 0.0 : rest4 <= kCus ? 0.70 : 1.10));
+  const int64_t rest8 = t8 % kCus, rounds = t8 / kCus;
+  const double eight = tile * ((t8 + kCus - 1) / kCus);
+  if (eight <= us) {
+    us = eight;
+    best = AttnPlan{8, (int)t8, 1};
+  }
+  us *= 0.90;
+  for (int64_t kp = 2; may_split && rest8 && kp <= kMaxParts && 4 * kp <= blocks; ++kp) {
+    const double t = tile * rounds + 1.85 * ((blocks + kp - 1) / kp) * ((rest8 * kp + kCus - 1) / kCus) + 5.0 +
+                     2.0 * rest8 * kp * kPart * 4 / 5e6;
+    if (t < us) {
+      us = t;
+      best = AttnPlan{8, (int)(t8 - rest8), (int)kp};
+    }
+  }
+  return best;
+}
+
+size_t attn_scratch_bytes(const AttnPlan &p, int64_t heads, int64_t rows) {
+  if (p.kparts < 2) return 0;
+  const int64_t tiles = heads * ((rows + 255) / 256) - p.full;
+  return (size_t)(tiles * p.kparts * kPart) * sizeof(float);
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -343,9 +470,22 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 }  // namespace
 }  // namespace mq
 
+extern "C" size_t mq_attention_scratch_size(int64_t batch, int heads, int64_t valid) {
+  using namespace mq;
+  if (batch <= 0 || heads <= 0 || valid <= 0) return 0;
+  const int64_t nb = batch < kMaxBatch ? batch : kMaxBatch, last = batch % kMaxBatch;
+  size_t n = attn_scratch_bytes(attn_plan(nb * heads, valid, valid, true), nb * heads, valid);
+  if (batch > kMaxBatch && last) {
+    const size_t m = attn_scratch_bytes(attn_plan(last * heads, valid, valid, true), last * heads, valid);
+    n = m > n ? m : n;
+  }
+  return n;
+}
+
 extern "C" int mq_attention_bf16(const void *q, const void *k, const void *v, int64_t batch, int heads,
                                  int64_t l_total, int head_dim, int64_t valid, const int64_t *drop, void *out,
-                                 int64_t out_batch_stride, int64_t ldo, float *lse, float *guard, void *stream) {
+                                 int64_t out_batch_stride, int64_t ldo, float *lse, float *guard, void *scratch,
+                                 size_t scratch_bytes, void *stream) {
   using namespace mq;
   auto invalid = [](const char *msg) { return set_error(MQ_E_INVALID, msg); };
   if (head_dim != kHd) return invalid("mq_attention_bf16: head_dim must be 128");
@@ -354,7 +494,8 @@ extern "C" int mq_attention_bf16(const void *q, const void *k, const void *v, in
   if (l_total > (int64_t(1) << 23) || batch * heads > (int64_t(1) << 20))
     return invalid("mq_attention_bf16: l_total above 2^23 or more than 2^20 heads");
   if (!q || !k || !v || !out) return invalid("mq_attention_bf16: NULL pointer");
-  if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out) || ldo % 8 || out_batch_stride % 8)
+  if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out) || !aligned16(scratch) || ldo % 8 ||
+      out_batch_stride % 8)
     return invalid("mq_attention_bf16: buffers must be 16-byte aligned, out's strides multiples of 8 elements");
   if (ldo < (int64_t)heads * kHd || out_batch_stride < 0) return invalid("mq_attention_bf16: bad out strides");
   for (int64_t b = 0; drop && b < batch; ++b)
@@ -374,17 +515,26 @@ extern "C" int mq_attention_bf16(const void *q, const void *k, const void *v, in
       keys.gap[i] = (int)gap;
       keys.npad[i] = (float)(l_total - valid + gap);
     }
-    auto launch = [&]<int W>() {
-      const int qtiles = (int)((valid + 32 * W - 1) / (32 * W));
-      hipLaunchKernelGGL((attention_kernel<W>), dim3((unsigned)(nb * heads * qtiles)), dim3(64 * W), 0,
-                         static_cast<hipStream_t>(stream), static_cast<const __bf16 *>(q) + b0 * hsize,
+    AttnPlan plan = attn_plan(nb * heads, valid, valid, scratch != nullptr);
+    if (attn_scratch_bytes(plan, nb * heads, valid) > scratch_bytes) plan = attn_plan(nb * heads, valid, valid, false);
+    auto launch = [&]<int W, bool kSplit>() {
+      const int qtiles = (int)((valid + 32 * W - 1) / (32 * W)), tiles = nb * heads * qtiles;
+      hipStream_t s = static_cast<hipStream_t>(stream);
+      __bf16 *o = static_cast<__bf16 *>(out) + b0 * out_batch_stride;
+      float *le = lse ? lse + b0 * heads * valid : nullptr, *part = static_cast<float *>(scratch);
+      unsigned int *gu = reinterpret_cast<unsigned int *>(guard);
+      hipLaunchKernelGGL((attention_kernel<W, kSplit>), dim3((unsigned)(plan.full + (tiles - plan.full) * plan.kparts)),
+                         dim3(64 * W), 0, s, static_cast<const __bf16 *>(q) + b0 * hsize,
                          static_cast<const __bf16 *>(k) + b0 * hsize, static_cast<const __bf16 *>(v) + b0 * hsize, heads,
-                         l_total, (int)valid, qtiles, keys, scale, static_cast<__bf16 *>(out) + b0 * out_batch_stride,
-                         out_batch_stride, ldo, lse ? lse + b0 * heads * valid : nullptr,
-                         reinterpret_cast<unsigned int *>(guard));
+                         l_total, (int)valid, qtiles, keys, scale, o, out_batch_stride, ldo, le, gu, plan.full,
+                         plan.kparts, part);
+      if constexpr (kSplit)
+        hipLaunchKernelGGL(combine_kernel, dim3(32, (unsigned)(tiles - plan.full)), dim3(256), 0, s, part,
+                           plan.kparts, plan.full, heads, (int)valid, qtiles, keys, o, out_batch_stride, ldo, le, gu);
     };
-    if (eight_waves(nb * heads, valid)) launch.template operator()<8>();
-    else launch.template operator()<4>();
+    if (plan.kparts > 1) launch.template operator()<8, true>();
+    else if (plan.waves == 8) launch.template operator()<8, false>();
+    else launch.template operator()<4, false>();
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(MQ_E_HIP, hipGetErrorString(e));
   }

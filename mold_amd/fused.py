@@ -129,11 +129,15 @@ def attention(q, k, v, valid: int, drops=None, out=None, lse=None, guard=None):
     drop = None
     if drops is not None and any(d is not None for d in drops):
         drop = (ctypes.c_int64 * (2 * b_))(*[x for d in drops for x in (d or (0, 0))])
+    lib = _lib.load()
     with torch.cuda.device(q.device):
-        check(_lib.load().mq_attention_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), b_, h, l, HEAD_DIM, valid, drop,
-                                            res.data_ptr(), res.stride(0) if res.dim() == 3 else 0, res.stride(-2),
-                                            lse.data_ptr() if lse is not None else None,
-                                            guard.data_ptr() if guard is not None else None, _stream_ptr()))
+        nbytes = lib.mq_attention_scratch_size(b_, h, valid)
+        scratch = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None   # freed to this stream
+        check(lib.mq_attention_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), b_, h, l, HEAD_DIM, valid, drop,
+                                    res.data_ptr(), res.stride(0) if res.dim() == 3 else 0, res.stride(-2),
+                                    lse.data_ptr() if lse is not None else None,
+                                    guard.data_ptr() if guard is not None else None,
+                                    scratch.data_ptr() if nbytes else None, nbytes, _stream_ptr()))
     if out is not None and res is not out:
         return out.copy_(res)
     return res

@@ -11,7 +11,7 @@ import pytest
 
 torch = pytest.importorskip("torch")
 
-from mold_amd import MoldqError
+from mold_amd import MoldqError, _lib
 from mold_amd import fused as FU
 from mold_amd.flux import PAD_MIN_SHARE, attention_bf16, attention_bf16_batch
 from tests.test_build_checks import HIPCC, _asm, _functions, _m0_outside_asm
@@ -55,8 +55,10 @@ def test_block_and_tile_edges(valid, heads):
 
 @gpu
 @pytest.mark.parametrize("heads,valid", [(40, 1664), (140, 512), (24, 2816)])
-def test_eight_wave_tiles_match_four_wave_tiles(heads, valid):
-    """Enough tiles for the 8-wave variant: each head equals the same head alone (4 waves) bit for bit."""
+def test_eight_wave_tiles_match_four_wave_tiles(heads, valid, monkeypatch):
+    """Enough tiles for the 8-wave variant: without scratch each head equals the same head alone (4 waves)
+    bit for bit."""
+    monkeypatch.setattr(_lib.load(), "mq_attention_scratch_size", lambda *a: 0)
     q, k, v = _inputs(1, heads, valid, valid)
     out = attention_bf16(q[0], k[0], v[0])
     for i in (0, heads // 2, heads - 1):
@@ -64,6 +66,34 @@ def test_eight_wave_tiles_match_four_wave_tiles(heads, valid):
         assert torch.equal(out[:, 128 * i:128 * i + 128], one)
     ref, _ = _ref(q[0, :1], k[0, :1], v[0, :1], valid)
     assert _err(out[:, :128], ref) < 3e-3
+
+
+@gpu
+@pytest.mark.parametrize("heads,valid,drop", [
+    (1, 2048, None), (1, 2049, (64, 1985)), (3, 2111, (0, 2110)), (2, 2560, (1, 2560)), (2, 4097, (100, 300)),
+    (12, 2816, None), (12, 3000, (1000, 1001))])
+def test_split_tiles(heads, valid, drop):
+    """Tiles whose keys are shared between workgroups: all of them (few heads) or those after whole rounds (12 heads x 2
+    elements), shares left empty by a masked range, remainders of rows and keys, the log-sum-exp and the guard."""
+    assert _lib.load().mq_attention_scratch_size(2, heads, valid) > 0
+    l = -(-valid // 256) * 256
+    q, k, v = _inputs(2, heads, l, valid, seed=13)
+    if drop is not None:
+        k[1, :, drop[0]:drop[1]] = 0
+        v[1, :, drop[0]:drop[1]] = 0
+    guard, lse = torch.zeros((), device="cuda"), torch.empty((2, heads, valid), device="cuda")
+    out = FU.attention(q, k, v, valid, drops=[None, drop], guard=guard, lse=lse)
+    assert torch.equal(out, FU.attention(q, k, v, valid, drops=[None, drop]))
+    share, hs = 0.0, sorted({0, heads - 1})
+    for b, d in ((0, None), (1, drop)):
+        n = l - valid + (0 if d is None else d[1] - d[0])
+        for h in hs:
+            ref, s = _ref(q[b, h:h + 1], k[b, h:h + 1], v[b, h:h + 1], valid, d)
+            assert _err(out[b, :, 128 * h:128 * h + 128], ref) < 3e-3, (b, h)
+            z = n + torch.exp(s[0]).sum(-1)
+            assert (lse[b, h].double().cpu() - z.log()).abs().max() < 1e-4, (b, h)
+            share = max(share, float((n / z).max()))
+    assert float(guard) >= share * (1 - 1e-4) and (len(hs) < heads or abs(float(guard) - share) <= 1e-4 * share)
 
 
 @gpu
@@ -148,12 +178,12 @@ def test_argument_checks():
     from mold_amd import _lib
     lib = _lib.load()
 
-    def call(hd=128, batch=1, heads=1, l=64, valid=64, drop=None, ldo=128, q=4096):
-        return lib.mq_attention_bf16(q, 4096, 4096, batch, heads, l, hd, valid, drop, 4096, 0, ldo, None, None, None)
+    def call(hd=128, batch=1, heads=1, l=64, valid=64, drop=None, ldo=128, q=4096, scratch=None):
+        return lib.mq_attention_bf16(q, 4096, 4096, batch, heads, l, hd, valid, drop, 4096, 0, ldo, None, None, scratch, 0, None)
     import ctypes
     rng = lambda *a: (ctypes.c_int64 * len(a))(*a)
     bad = [dict(hd=64), dict(valid=65), dict(heads=0), dict(ldo=120), dict(ldo=132), dict(q=4100), dict(q=0), dict(batch=-1),
-           dict(drop=rng(0, 64)), dict(drop=rng(5, 3)), dict(drop=rng(-1, 3)), dict(drop=rng(1, 65)), dict(l=1 << 24)]
+           dict(drop=rng(0, 64)), dict(drop=rng(5, 3)), dict(drop=rng(-1, 3)), dict(drop=rng(1, 65)), dict(l=1 << 24), dict(scratch=4100)]
     for kw in bad:
         assert call(**kw) == -1, kw
         with pytest.raises(MoldqError):
@@ -165,7 +195,7 @@ def test_argument_checks():
 @pytest.mark.skipif(HIPCC is None, reason="hipcc not available")
 def test_kernel_leaves_m0_alone_and_does_not_spill(tmp_path):
     funcs = {k: v for k, v in _functions(_asm(tmp_path, "mq_attn.hip")).items() if "attention_kernel" in k}
-    assert len(funcs) == 2
+    assert len(funcs) == 3
     for name, (lines, meta) in funcs.items():
         assert not _m0_outside_asm(lines), name
         assert meta.get("ScratchSize", 0) == 0, (name, meta)
