@@ -61,6 +61,8 @@ def _m0_outside_asm(lines):
 
 @pytest.mark.parametrize("src,defines,kernel", [
     ("mq_gemm.hip", ("MQ_GEMM_TYPE=Q4_K",), "gemm_fast_kernel"),
+    ("mq_gemm.hip", ("MQ_GEMM_TYPE=Q8_0",), "gemm_skinny_kernel"),
+    ("mq_gemm.hip", ("MQ_GEMM_TYPE=Q6_K",), "gemm_skinny_kernel"),
     ("mq_gemv.hip", (), "gemv_q4k_kernel"),
 ])
 def test_lds_dma_kernels_leave_m0_alone_and_do_not_spill(tmp_path, src, defines, kernel):
