@@ -775,8 +775,7 @@ def bench_flux(dev, args):
            "flop_linear": lin, "flop_attention": attn,
            "weight_bytes": params.quantized_bytes(), "attention": F.ATTENTION_BACKEND["name"],
            "config": "FLUX.1-dev shape, 1024x1024, batch 1, 4096 img + 512 txt tokens, Q4_K linears, "
-                     "f32 activations, bf16 GEMM inputs and attention; attention is PyTorch's fused SDPA "
-                     "(on ROCm AOTriton's precompiled attn_fwd kernel), not part of libmoldq"}
+                     "f32 activations, bf16 GEMM inputs and attention (mq_attention_bf16)"}
     return res, params, inp
 
 
@@ -843,9 +842,8 @@ def bench_qwen(dev, args):
            "weight_bytes": params.quantized_bytes(), "attention": ATTENTION_BACKEND["name"],
            "config": f"Qwen-Image shape, 1328x1328, batch 1, {l_img} img + 256 txt tokens, 60 blocks; "
                      "q/k/v Q3_K (stacked per stream), MLP Q2_K, out-projections, modulation, stems Q4_K; "
-                     "f32 residuals, bf16 GEMM inputs and attention (joint sequence padded to a multiple of 256 "
-                     "with zero keys, corrected by the log-sum-exp), text stream on a second HIP stream; attention is "
-                     "PyTorch's fused SDPA (on ROCm AOTriton's precompiled attn_fwd kernel), not part of libmoldq"}
+                     "f32 residuals, bf16 GEMM inputs and attention (mq_attention_bf16; joint buffers padded to a "
+                     "multiple of 256), text stream on a second HIP stream"}
     return res, params, inp
 
 
