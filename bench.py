@@ -518,7 +518,7 @@ def bench_encoder_decode(dev, args):
             torch.cuda.empty_cache()
     return {"t5_encoder_m512": enc, "small_m_gemm": mid, "decode_gemv_m1": dec,
             "what": "T5-XXL encoder linears (f32 x staged to bf16 + fused GEMM) at M=512; small-m GEMMs "
-                    "(64- / 128-row tiles) at M=77 and 256; LLM-decode M=1 GEMVs "
+                    "(32- to 128-row tiles) at M=77 and 256; LLM-decode M=1 GEMVs "
                     "(f32 x; Q4_K takes the Q8_K integer-dot GEMV, other types the f32-FMA GEMV)"}
 
 
@@ -550,7 +550,7 @@ def bench_lora(dev, args):
     torch.cuda.synchronize()
     dev_ms = (time.perf_counter() - t0) * 1e3 / reps
     res = {"weight": "Q4_K", "n": n, "k": k, "rank": rank, "patches": applied, "device_ms": round(dev_ms, 2),
-           "what": "mq_dequantize + 4 mq_lora_apply (Q, K, V 3072 rows, MLP 12288 rows) + mq_quantize (ggml "
+           "what": "mq_lora_merge of 4 patches (Q, K, V 3072 rows, MLP 12288 rows; requantized by the ggml "
                    "reference Q4_K quantizer), synchronous"}
     if not args.no_cpu:
         from oracle import oracle as O
