@@ -369,9 +369,8 @@ def attention_bf16(q, k, v, valid: Optional[int] = None, guard=None, drop: Optio
     zero, so they are removed by the same correction (n_pad counts them too).
 
     `out`, a bf16 [valid, H*D] tensor whose rows may be strided (a column block
-    of a wider buffer), receives the result in place of a new tensor: the
-    correction pass writes it there, the unpadded path copies its [H, L, D]
-    output there once.
+    of a wider buffer), receives the result in place of a new tensor.  It may be on
+    another device where nothing is padded or masked.
 
     Where no fused kernel serves the device, it falls back to the exact
     head-chunked path on the valid rows (any other error propagates).  The
@@ -387,6 +386,8 @@ def attention_bf16(q, k, v, valid: Optional[int] = None, guard=None, drop: Optio
     if ATTENTION_BACKEND["name"] in (None, "fused") and 0 < valid <= l and _drop_ok(drop, valid) \
             and (guard is None or guard.is_cuda) and takes_attention(qb, kb, vb):
         ATTENTION_BACKEND["name"] = "fused"
+        if out is not None and out.device != q.device and (valid < l or n_drop):
+            raise ValueError("attention_bf16: a padded call's out must be on q's device")
         if guard is not None or not (valid < l or n_drop):
             return attention(qb, kb, vb, valid, drops=[drop], out=out, guard=guard if valid < l or n_drop else None)
         lse = torch.empty((1, h, valid), dtype=torch.float32, device=q.device)

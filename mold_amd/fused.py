@@ -117,14 +117,14 @@ def attention(q, k, v, valid: int, drops=None, out=None, lse=None, guard=None):
     """softmax(q k^T / sqrt(128)) v over rows and keys 0 .. valid-1 of bf16 [B, H, L, 128]
     (or [H, L, 128]), element b's keys drops[b] = (lo, hi) masked out (mq_attention_bf16).
     Returns bf16 [B, valid, H*128] ([valid, H*128]): `out` when given (unit column stride;
-    written through a temporary if its rows are not 16-byte aligned).  lse f32 [B, H, valid]
+    written through a temporary if it is on another device or its rows are not 16-byte aligned).  lse f32 [B, H, valid]
     and guard (0-dim f32, raised) as mq_attention_bf16 describes them."""
     import torch
     b_ = q.shape[0] if q.dim() == 4 else 1
     h, l = q.shape[-3], q.shape[-2]
     shape = (b_, valid, h * HEAD_DIM) if q.dim() == 4 else (valid, h * HEAD_DIM)
     res = out
-    if out is None or out.data_ptr() % 16 or any(s % 8 for s in out.stride()[:-1]):
+    if out is None or out.device != q.device or out.data_ptr() % 16 or any(s % 8 for s in out.stride()[:-1]):
         res = torch.empty(shape, dtype=torch.bfloat16, device=q.device)
     drop = None
     if drops is not None and any(d is not None for d in drops):

@@ -158,6 +158,18 @@ def test_lse_and_strided_out():
 
 
 @gpu
+def test_out_on_the_host():
+    """Filled by a copy where nothing is padded, refused where something is."""
+    q, k, v = (t[0] for t in _inputs(1, 2, 96, 96, seed=17))
+    host = torch.empty((96, 256), dtype=torch.bfloat16)
+    assert attention_bf16(q, k, v, out=host) is host
+    assert torch.equal(host, attention_bf16(q, k, v).cpu())
+    for guard in (None, torch.zeros((), device="cuda")):
+        with pytest.raises(ValueError):
+            attention_bf16(q, k, v, valid=90, guard=guard, out=host[:90])
+
+
+@gpu
 def test_other_calls_keep_pytorch_attention():
     """Inputs that autograd records, other head sizes and non-contiguous or mixed inputs do not take the kernel and still work."""
     q, k, v = (t[0] for t in _inputs(1, 2, 64, 64, seed=13))
