@@ -283,7 +283,8 @@ int mq_attn_pad_correct(const void *o, int64_t batch, int heads, int64_t rows, i
  * and the l_total - valid + hi - lo padded and masked ones counted as zero
  * scores; *guard (f32 >= 0, or NULL) is raised to the largest share of a
  * row's mass those zero scores would hold (what mq_attn_pad_correct reports).
- * Buffers 16-byte aligned, out's strides multiples of 8 elements.  Replaces
+ * Buffers 16-byte aligned, out's strides multiples of 8 elements, and out,
+ * from its first row to its last, clear of q, k and v.  Replaces
  * attention() at crates/mold-inference/src/flux/offload.rs:39-54 and
  * crates/mold-inference/src/qwen_image/quantized_transformer.rs:804-823.
  * Asynchronous on stream. */

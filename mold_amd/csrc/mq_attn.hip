@@ -503,6 +503,13 @@ extern "C" int mq_attention_bf16(const void *q, const void *k, const void *v, in
         drop[2 * b + 1] - drop[2 * b] >= (valid > 0 ? valid : 1))
       return invalid("mq_attention_bf16: a masked range must lie in 0 .. valid and leave a key");
   if (batch == 0 || valid == 0) return MQ_OK;
+  // a tile's rows are stored while other workgroups still read q, k and v
+  const uintptr_t in_bytes = (uintptr_t)(batch * heads * l_total * kHd) * 2, o0 = reinterpret_cast<uintptr_t>(out);
+  const uintptr_t o1 = o0 + (uintptr_t)((batch - 1) * out_batch_stride + (valid - 1) * ldo + heads * (int64_t)kHd) * 2;
+  for (const void *in : {q, k, v}) {
+    const uintptr_t i0 = reinterpret_cast<uintptr_t>(in);
+    if (o0 < i0 + in_bytes && i0 < o1) return invalid("mq_attention_bf16: out lies over q, k or v");
+  }
   const int64_t hsize = heads * l_total * kHd;
   const float scale = 0.12751743f;  // log2(e) / sqrt(128)
   for (int64_t b0 = 0; b0 < batch; b0 += kMaxBatch) {

@@ -369,14 +369,14 @@ def attention_bf16(q, k, v, valid: Optional[int] = None, guard=None, drop: Optio
     zero, so they are removed by the same correction (n_pad counts them too).
 
     `out`, a bf16 [valid, H*D] tensor whose rows may be strided (a column block
-    of a wider buffer), receives the result in place of a new tensor.  It may be on
-    another device where nothing is padded or masked.
+    of a wider buffer), receives the result in place of a new tensor.  It may lie over
+    q, k or v, and on another device where nothing is padded or masked.
 
     Where no fused kernel serves the device, it falls back to the exact
     head-chunked path on the valid rows (any other error propagates).  The
     backend used is recorded in ATTENTION_BACKEND."""
     import torch
-    from .fused import attention, takes_attention
+    from .fused import apart, attention, takes_attention
     h, l, d = q.shape
     valid = l if valid is None else valid
     qb, kb, vb = (t.to(torch.bfloat16).contiguous() for t in (q, k, v))
@@ -391,13 +391,15 @@ def attention_bf16(q, k, v, valid: Optional[int] = None, guard=None, drop: Optio
         if guard is not None or not (valid < l or n_drop):
             return attention(qb, kb, vb, valid, drops=[drop], out=out, guard=guard if valid < l or n_drop else None)
         lse = torch.empty((1, h, valid), dtype=torch.float32, device=q.device)
-        res = attention(qb, kb, vb, valid, drops=[drop], out=out, lse=lse)
+        # a recompute reads q, k and v again
+        dst = out if out is None or apart(out, qb, kb, vb) else None
+        res = attention(qb, kb, vb, valid, drops=[drop], out=dst, lse=lse)
         bad = ((l - valid + n_drop) * torch.exp(-lse[0]) > 1.0 - PAD_MIN_SHARE).any(dim=1)
         if bool(bad.any()):
             heads = bad.nonzero().flatten()
             exact = _attention_chunked(qb[heads, :valid], kb[heads, :valid], vb[heads, :valid], drop)
             res.view(valid, h, d)[:, heads] = exact.view(valid, heads.numel(), d)
-        return res
+        return res if out is dst else out.copy_(res)
     if ATTENTION_BACKEND["name"] in (None, "fused"):
         try:
             if valid < l or n_drop:

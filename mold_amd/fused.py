@@ -113,18 +113,29 @@ def takes_attention(q, k, v) -> bool:
             and torch._C._len_torch_dispatch_stack() == 0 and not torch.compiler.is_compiling())
 
 
+def apart(out, *inputs) -> bool:
+    """Whether out's bytes, first to last, lie clear of the (contiguous) inputs'."""
+    size = out.element_size()
+    lo = out.data_ptr()
+    hi = lo + size * (1 + sum((n - 1) * st for n, st in zip(out.shape, out.stride())))
+    return all(t.device != out.device or hi <= t.data_ptr() or t.data_ptr() + t.numel() * t.element_size() <= lo
+               for t in inputs)
+
+
 def attention(q, k, v, valid: int, drops=None, out=None, lse=None, guard=None):
     """softmax(q k^T / sqrt(128)) v over rows and keys 0 .. valid-1 of bf16 [B, H, L, 128]
     (or [H, L, 128]), element b's keys drops[b] = (lo, hi) masked out (mq_attention_bf16).
     Returns bf16 [B, valid, H*128] ([valid, H*128]): `out` when given (unit column stride;
-    written through a temporary if it is on another device or its rows are not 16-byte aligned).  lse f32 [B, H, valid]
+    written through a temporary if it is on another device, its rows are not 16-byte aligned or
+    it lies over q, k or v, which other workgroups still read when a tile's rows are stored).  lse f32 [B, H, valid]
     and guard (0-dim f32, raised) as mq_attention_bf16 describes them."""
     import torch
     b_ = q.shape[0] if q.dim() == 4 else 1
     h, l = q.shape[-3], q.shape[-2]
     shape = (b_, valid, h * HEAD_DIM) if q.dim() == 4 else (valid, h * HEAD_DIM)
     res = out
-    if out is None or out.device != q.device or out.data_ptr() % 16 or any(s % 8 for s in out.stride()[:-1]):
+    if out is None or out.device != q.device or out.data_ptr() % 16 or any(s % 8 for s in out.stride()[:-1]) \
+            or not apart(out, q, k, v):
         res = torch.empty(shape, dtype=torch.bfloat16, device=q.device)
     drop = None
     if drops is not None and any(d is not None for d in drops):

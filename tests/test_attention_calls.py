@@ -25,6 +25,7 @@ class _Lib:
 
     def __init__(self):
         self.calls = []
+        self.fill_lse = None     # a head's log-sum-exp
 
     def mq_attention_scratch_size(self, *a):
         return 0
@@ -32,6 +33,9 @@ class _Lib:
     def mq_attention_bf16(self, q, k, v, batch, heads, l, hd, valid, drop, out, sb, ldo, lse, guard, *_):
         self.calls.append(types.SimpleNamespace(out=out, ldo=ldo, lse=lse, guard=guard))
         assert hd == HD and ldo >= heads * HD
+        if lse and self.fill_lse is not None:
+            _at(lse, heads * valid, torch.float32, ctypes.c_float).view(heads, valid).copy_(
+                self.fill_lse[:, None].expand(heads, valid))
         for b in range(batch):
             for h in range(heads):
                 qh, kh, vh = (_at(p + 2 * HD * l * (b * heads + h), l * HD).view(l, HD) for p in (q, k, v))
@@ -68,3 +72,54 @@ def test_out_on_another_device(lib):
     with pytest.raises(ValueError):
         F.attention_bf16(q, k, v, valid=L - 3, out=out[:L - 3])
     assert len(lib.calls) == 1 and lib.calls[0].out
+
+
+def _reference(q, k, v, valid=L):
+    s = q[:, :valid].float() @ k[:, :valid].float().transpose(1, 2) / math.sqrt(HD)
+    return (torch.softmax(s, -1) @ v[:, :valid].float()).transpose(0, 1).reshape(valid, H * HD)
+
+
+@pytest.mark.parametrize("over", ["q", "k", "v", "q and k"])
+@pytest.mark.parametrize("padded", [False, True])
+def test_out_over_its_inputs(lib, over, padded):
+    """q, k and v are read whole before out changes; a recomputed head (the scores of head 1 are all
+    below -10 over the padding's 0) reads them too."""
+    qkv = _qkv()
+    valid = L - 5 if padded else L
+    if padded:
+        qkv[1, 1] = -qkv[0, 1, :1] * 4
+        qkv[0, 1] = qkv[0, 1, :1]
+        qkv[1:, :, valid:] = 0
+    q, k, v = qkv
+    ref = _reference(q, k, v, valid)
+    at = {"q": 0, "k": 1, "v": 2, "q and k": 0.5}[over]
+    flat = qkv.view(-1)
+    out = flat[int(at * q.numel()):][:valid * H * HD].view(valid, H * HD)
+    if padded:
+        lib.fill_lse = torch.tensor([50.0, -50.0])
+    assert F.attention_bf16(q, k, v, valid=valid, out=out) is out
+    assert ((out.float() - ref).norm() / ref.norm()).item() < 6e-3     # two roundings to bf16
+    assert all(c.out != out.data_ptr() for c in lib.calls)
+
+
+def test_a_separate_out_is_written_directly(lib):
+    q, k, v = _qkv()
+    wide = torch.full((L, H * HD + 16), 3.0, dtype=torch.bfloat16)
+    out = wide[:, 8:8 + H * HD]
+    assert F.attention_bf16(q, k, v, out=out) is out and lib.calls[0].out == out.data_ptr()
+    ref = _reference(q, k, v)
+    assert ((out.float() - ref).norm() / ref.norm()).item() < 6e-3
+    assert bool((wide[:, :8] == 3.0).all()) and bool((wide[:, 8 + H * HD:] == 3.0).all())
+
+
+@pytest.mark.parametrize("at", [-1, 0, 3])
+def test_c_entry_refuses_out_over_its_inputs(at):
+    """Addresses only: the refusal comes before any launch."""
+    from mold_amd import _lib
+    base, size = 1 << 20, 64 * HD * 2
+    ins = [base, base + 4 * size, base + 8 * size]
+    for i in range(3):
+        args = list(ins)
+        out = args[i] + at * size // 4
+        rc = _lib.load().mq_attention_bf16(*args, 1, 1, 64, HD, 64, None, out, 0, HD, None, None, None, 0, None)
+        assert rc == -1 and b"lies over" in _lib.load().mq_last_error()
