@@ -384,7 +384,7 @@ def attention_bf16(q, k, v, valid: Optional[int] = None, guard=None, drop: Optio
     if out is not None and (out.shape != (valid, h * d) or out.dtype != torch.bfloat16 or out.stride(1) != 1):
         raise ValueError(f"attention_bf16: out must be bf16 [{valid}, {h * d}] with unit column stride")
     if ATTENTION_BACKEND["name"] in (None, "fused") and 0 < valid <= l and _drop_ok(drop, valid) \
-            and (guard is None or guard.is_cuda) and takes_attention(qb, kb, vb):
+            and takes_attention(qb, kb, vb):
         ATTENTION_BACKEND["name"] = "fused"
         if out is not None and out.device != q.device and (valid < l or n_drop):
             raise ValueError("attention_bf16: a padded call's out must be on q's device")
@@ -481,10 +481,11 @@ def attention_bf16_batch(q, k, v, valid: int, guard, drops):
                                        for b in range(b_)])
     if guard is None or ATTENTION_BACKEND["name"] not in (None, "fused"):
         return per_element()
-    from .fused import attention, takes_attention
-    if 0 < valid <= l and all(_drop_ok(dr, valid) for dr in drops) and len(drops) == b_ and guard.is_cuda \
+    from .fused import attention, check_guard, takes_attention
+    if 0 < valid <= l and all(_drop_ok(dr, valid) for dr in drops) and len(drops) == b_ \
             and takes_attention(q, k, v):
         ATTENTION_BACKEND["name"] = "fused"
+        check_guard(guard, q.device)
         padded = valid < l or any(dr is not None and dr[1] > dr[0] for dr in drops)
         return attention(q, k, v, valid, drops=drops, guard=guard if padded else None)
     try:

@@ -122,17 +122,32 @@ def apart(out, *inputs) -> bool:
                for t in inputs)
 
 
+def check_guard(guard, device):
+    """The kernels raise a guard with a 4-byte atomic at its address."""
+    import torch
+    if guard.dtype != torch.float32 or guard.numel() != 1 or guard.device != device:
+        raise ValueError("attention: guard must be a one-element f32 tensor on q's device")
+
+
 def attention(q, k, v, valid: int, drops=None, out=None, lse=None, guard=None):
     """softmax(q k^T / sqrt(128)) v over rows and keys 0 .. valid-1 of bf16 [B, H, L, 128]
-    (or [H, L, 128]), element b's keys drops[b] = (lo, hi) masked out (mq_attention_bf16).
-    Returns bf16 [B, valid, H*128] ([valid, H*128]): `out` when given (unit column stride;
-    written through a temporary if it is on another device, its rows are not 16-byte aligned or
-    it lies over q, k or v, which other workgroups still read when a tile's rows are stored).  lse f32 [B, H, valid]
-    and guard (0-dim f32, raised) as mq_attention_bf16 describes them."""
+    (or [H, L, 128]) that `takes_attention` accepts, element b's keys drops[b] = (lo, hi) masked
+    out (mq_attention_bf16).  Returns bf16 [B, valid, H*128] ([valid, H*128]): `out` when given
+    (unit column stride; written through a temporary if it is on another device, its rows are
+    not 16-byte aligned or it lies over q, k or v, which other workgroups still read when a
+    tile's rows are stored).  lse f32 [B, H, valid] and guard (one f32, raised) as
+    mq_attention_bf16 describes them."""
     import torch
     b_ = q.shape[0] if q.dim() == 4 else 1
     h, l = q.shape[-3], q.shape[-2]
     shape = (b_, valid, h * HEAD_DIM) if q.dim() == 4 else (valid, h * HEAD_DIM)
+    if out is not None and (out.dtype != torch.bfloat16 or tuple(out.shape) != shape or out.stride(-1) != 1):
+        raise ValueError(f"attention: out must be bf16 {list(shape)} with unit column stride")
+    if guard is not None:
+        check_guard(guard, q.device)
+    if lse is not None and (lse.dtype != torch.float32 or tuple(lse.shape) != (b_, h, valid) or not lse.is_contiguous()
+                            or lse.device != q.device):
+        raise ValueError(f"attention: lse must be contiguous f32 {[b_, h, valid]} on q's device")
     res = out
     if out is None or out.device != q.device or out.data_ptr() % 16 or any(s % 8 for s in out.stride()[:-1]) \
             or not apart(out, q, k, v):

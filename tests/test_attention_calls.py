@@ -123,3 +123,33 @@ def test_c_entry_refuses_out_over_its_inputs(at):
         out = args[i] + at * size // 4
         rc = _lib.load().mq_attention_bf16(*args, 1, 1, 64, HD, 64, None, out, 0, HD, None, None, None, 0, None)
         assert rc == -1 and b"lies over" in _lib.load().mq_last_error()
+
+
+@pytest.mark.parametrize("guard", [torch.zeros((), dtype=torch.bfloat16), torch.zeros((), dtype=torch.float64), torch.zeros(2),
+                                   torch.zeros((), device="meta")], ids=["bf16", "f64", "two", "elsewhere"])
+def test_a_guard_the_kernel_cannot_raise(lib, guard):
+    """Refused where the call is padded or batched, not looked at in an unpadded single one."""
+    q, k, v = _qkv()
+    for call in (lambda: F.attention_bf16(q, k, v, valid=L - 1, guard=guard),
+                 lambda: F.attention_bf16_batch(q[None], k[None], v[None], L - 1, guard, [None]),
+                 lambda: F.attention_bf16_batch(q[None], k[None], v[None], L, guard, [None])):
+        with pytest.raises(ValueError):
+            call()
+    assert not lib.calls
+    assert F.attention_bf16(q, k, v, guard=guard).shape == (L, H * HD) and lib.calls[0].guard is None
+    one = torch.zeros((1, 1))
+    F.attention_bf16(q, k, v, valid=L - 1, guard=one)
+    assert lib.calls[1].guard == one.data_ptr()
+
+
+def test_an_lse_or_out_the_kernel_cannot_write(lib):
+    q, k, v = _qkv()
+    for lse in (torch.empty((1, H, L), dtype=torch.bfloat16), torch.empty((1, H, L - 1)), torch.empty((1, H, 2 * L))[:, :, ::2],
+                torch.empty((1, H, L), device="meta")):
+        with pytest.raises(ValueError):
+            FU.attention(q, k, v, L, lse=lse)
+    for out in (torch.empty((L, H * HD)), torch.empty((L - 1, H * HD), dtype=torch.bfloat16),
+                torch.empty((H * HD, L), dtype=torch.bfloat16).t()):
+        with pytest.raises(ValueError):
+            FU.attention(q, k, v, L, out=out)
+    assert not lib.calls
