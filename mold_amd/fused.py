@@ -95,22 +95,28 @@ def attn_pad_correct(o, lse, npad, rows: int, guard, out):
     return out
 
 
+def recorded(*inputs) -> bool:
+    """Whether something records or interprets the call (autograd, a functorch transform,
+    forward-mode AD, a dispatch mode, a compiler, a trace): it needs operations PyTorch
+    knows."""
+    import torch
+    return ((torch.is_grad_enabled() and any(t.requires_grad for t in inputs))
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._len_torch_dispatch_stack() != 0 or torch.compiler.is_compiling()
+            or torch.jit.is_tracing())
+
+
 def takes_attention(q, k, v) -> bool:
     """Whether `attention` computes these q, k, v: bf16 [.., H, L, 128] of one shape on one
-    GPU, contiguous and 16-byte aligned, with nothing recording the call (autograd, a
-    functorch transform, forward-mode AD, a dispatch mode, a compiler): those need
-    operations PyTorch knows."""
+    GPU, contiguous and 16-byte aligned, with nothing recording the call."""
     import torch
     for t in (q, k, v):
         if type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda or t.dtype != torch.bfloat16 \
                 or t.shape != q.shape or t.device != q.device or not t.is_contiguous() or t.data_ptr() % 16:
             return False
-        if t.requires_grad and torch.is_grad_enabled():
-            return False
     return (q.dim() in (3, 4) and q.shape[-1] == HEAD_DIM and 0 < q.numel() and q.shape[-2] <= 1 << 23
-            and torch._C._functorch.peek_interpreter_stack() is None
-            and torch.autograd.forward_ad._current_level < 0
-            and torch._C._len_torch_dispatch_stack() == 0 and not torch.compiler.is_compiling())
+            and not recorded(q, k, v))
 
 
 def apart(out, *inputs) -> bool:

@@ -31,6 +31,7 @@ class _Lib:
         return 0
 
     def mq_attention_bf16(self, q, k, v, batch, heads, l, hd, valid, drop, out, sb, ldo, lse, guard, *_):
+        batch, heads, l, valid, sb, ldo = map(int, (batch, heads, l, valid, sb, ldo))     # a trace's sizes are tensors
         self.calls.append(types.SimpleNamespace(out=out, ldo=ldo, lse=lse, guard=guard))
         assert hd == HD and ldo >= heads * HD
         if lse and self.fill_lse is not None:
@@ -47,14 +48,20 @@ class _Lib:
         return 0
 
 
+def _efficient(q, k, v, bias, want_lse):
+    s = q.float() @ k.float().transpose(-1, -2) / math.sqrt(HD)
+    return (torch.softmax(s, -1) @ v.float()).to(q.dtype), torch.logsumexp(s, -1)
+
+
 @pytest.fixture
 def lib(monkeypatch):
     fake = _Lib()
     monkeypatch.setattr(FU._lib, "load", lambda *a: fake)
     monkeypatch.setattr(FU, "_stream_ptr", lambda *a: 0)
-    monkeypatch.setattr(FU, "takes_attention", lambda q, k, v: True)
+    monkeypatch.setattr(FU, "takes_attention", lambda q, k, v: not FU.recorded(q, k, v))
     monkeypatch.setattr(torch.cuda, "device", lambda d: contextlib.nullcontext())
     monkeypatch.setattr(F, "ATTENTION_BACKEND", {"name": None})
+    monkeypatch.setattr(torch.ops.aten, "_scaled_dot_product_efficient_attention", _efficient)    # not on the CPU
     return fake
 
 
@@ -153,3 +160,13 @@ def test_an_lse_or_out_the_kernel_cannot_write(lib):
         with pytest.raises(ValueError):
             FU.attention(q, k, v, L, out=out)
     assert not lib.calls
+
+
+def test_a_traced_call_replays(lib):
+    """torch.jit.trace: the kernel's call would leave only the allocation of its result in the graph."""
+    q, k, v = _qkv()
+    traced = torch.jit.trace(lambda a, b, c: F.attention_bf16(a, b, c), (q, k, v), check_trace=False)
+    assert not lib.calls
+    x, y, z = (t.flip(1).contiguous() for t in (q, k, v))
+    ref = _reference(x, y, z)
+    assert ((traced(x, y, z).float() - ref).norm() / ref.norm()).item() < 6e-3
