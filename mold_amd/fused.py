@@ -95,16 +95,23 @@ def attn_pad_correct(o, lse, npad, rows: int, guard, out):
     return out
 
 
+def _recording_mode() -> bool:
+    """A torch function mode other than the device context, which changes factory calls only."""
+    from torch.overrides import _get_current_function_mode_stack
+    from torch.utils._device import DeviceContext
+    return any(not isinstance(m, DeviceContext) for m in _get_current_function_mode_stack())
+
+
 def recorded(*inputs) -> bool:
     """Whether something records or interprets the call (autograd, a functorch transform,
-    forward-mode AD, a dispatch mode, a compiler, a trace): it needs operations PyTorch
-    knows."""
+    forward-mode AD, a dispatch or function mode, a compiler, a trace): it needs operations
+    PyTorch knows."""
     import torch
     return ((torch.is_grad_enabled() and any(t.requires_grad for t in inputs))
             or torch._C._functorch.peek_interpreter_stack() is not None
             or torch.autograd.forward_ad._current_level >= 0
             or torch._C._len_torch_dispatch_stack() != 0 or torch.compiler.is_compiling()
-            or torch.jit.is_tracing())
+            or torch.jit.is_tracing() or (torch._C._is_torch_function_mode_enabled() and _recording_mode()))
 
 
 def takes_attention(q, k, v) -> bool:

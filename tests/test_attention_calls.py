@@ -170,3 +170,27 @@ def test_a_traced_call_replays(lib):
     x, y, z = (t.flip(1).contiguous() for t in (q, k, v))
     ref = _reference(x, y, z)
     assert ((traced(x, y, z).float() - ref).norm() / ref.norm()).item() < 6e-3
+
+
+def test_a_function_mode_sees_the_operations(lib):
+    """A mode that records functions gets PyTorch's; the one that torch.device(..) pushes records nothing."""
+    from torch.overrides import TorchFunctionMode
+
+    class Names(TorchFunctionMode):
+        seen = []
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.seen.append(getattr(func, "__name__", str(func)))
+            return func(*args, **(kwargs or {}))
+    q, k, v = _qkv()
+    with Names():
+        F.attention_bf16(q, k, v)
+    assert not lib.calls and "softmax" in Names.seen
+    with torch.device("cpu"):
+        F.attention_bf16(q, k, v)
+    assert len(lib.calls) == 1
+    with Names(), torch.device("cpu"):
+        F.attention_bf16(q, k, v)
+    with Names(), torch._C.DisableTorchFunction():
+        F.attention_bf16(q, k, v)
+    assert len(lib.calls) == 2
