@@ -287,7 +287,8 @@ class QMatMul:
             x_data = x if len(lead) == 1 else x.reshape(-1, k)
             if x_data.stride(1) != 1:
                 x_data = x_data.contiguous()
-            m, ldx = x_data.shape[0], x_data.stride(0)
+            m = x_data.shape[0]
+            ldx = k if m == 1 else x_data.stride(0)     # one row may have any stride
             if out_dtype is None:
                 out_dtype = out.dtype if out is not None else x.dtype
             x_code = _dtype_code(x_data.dtype)
