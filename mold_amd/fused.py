@@ -161,10 +161,13 @@ def attention(q, k, v, valid: int, drops=None, out=None, lse=None, guard=None):
     if lse is not None and (lse.dtype != torch.float32 or tuple(lse.shape) != (b_, h, valid) or not lse.is_contiguous()
                             or lse.device != q.device):
         raise ValueError(f"attention: lse must be contiguous f32 {[b_, h, valid]} on q's device")
+    # row and batch stride, read only where there is more than one
+    ldo = out.stride(-2) if out is not None and valid > 1 else h * HEAD_DIM
+    sb = out.stride(0) if out is not None and b_ > 1 else valid * ldo
     res = out
-    if out is None or out.device != q.device or out.data_ptr() % 16 or any(s % 8 for s in out.stride()[:-1]) \
-            or not apart(out, q, k, v):
+    if out is None or out.device != q.device or out.data_ptr() % 16 or ldo % 8 or sb % 8 or not apart(out, q, k, v):
         res = torch.empty(shape, dtype=torch.bfloat16, device=q.device)
+        ldo, sb = h * HEAD_DIM, valid * h * HEAD_DIM
     drop = None
     if drops is not None and any(d is not None for d in drops):
         drop = (ctypes.c_int64 * (2 * b_))(*[x for d in drops for x in (d or (0, 0))])
@@ -173,7 +176,7 @@ def attention(q, k, v, valid: int, drops=None, out=None, lse=None, guard=None):
         nbytes = lib.mq_attention_scratch_size(b_, h, valid)
         scratch = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None   # freed to this stream
         check(lib.mq_attention_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), b_, h, l, HEAD_DIM, valid, drop,
-                                    res.data_ptr(), res.stride(0) if res.dim() == 3 else 0, res.stride(-2),
+                                    res.data_ptr(), sb, ldo,
                                     lse.data_ptr() if lse is not None else None,
                                     guard.data_ptr() if guard is not None else None,
                                     scratch.data_ptr() if nbytes else None, nbytes, _stream_ptr()))

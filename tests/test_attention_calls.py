@@ -194,3 +194,15 @@ def test_a_function_mode_sees_the_operations(lib):
     with Names(), torch._C.DisableTorchFunction():
         F.attention_bf16(q, k, v)
     assert len(lib.calls) == 2
+
+
+def test_one_row_of_out_may_have_any_stride(lib):
+    """A dimension of one has any stride; the library takes ldo >= H * 128."""
+    q, k, v = (t[:, :1].contiguous() for t in _qkv())
+    ref = v.transpose(0, 1).reshape(1, H * HD)
+    for stride in (0, 1, 8, H * HD + 4):
+        out = torch.empty(2 * H * HD, dtype=torch.bfloat16).as_strided((1, H * HD), (stride, 1))
+        assert F.attention_bf16(q, k, v, out=out) is out and torch.equal(out, ref)
+    one = torch.empty((1, H * HD), dtype=torch.bfloat16).as_strided((1, 1, H * HD), (3, 5, 1))
+    assert torch.equal(FU.attention(q[None], k[None], v[None], 1, out=one)[0], ref)
+    assert [c.ldo for c in lib.calls] == [H * HD] * 5
