@@ -376,7 +376,7 @@ def attention_bf16(q, k, v, valid: Optional[int] = None, guard=None, drop: Optio
     head-chunked path on the valid rows (any other error propagates).  The
     backend used is recorded in ATTENTION_BACKEND."""
     import torch
-    from .fused import apart, attention, takes_attention
+    from .fused import apart, attention, recorded, takes_attention
     h, l, d = q.shape
     valid = l if valid is None else valid
     qb, kb, vb = (t.to(torch.bfloat16).contiguous() for t in (q, k, v))
@@ -384,7 +384,7 @@ def attention_bf16(q, k, v, valid: Optional[int] = None, guard=None, drop: Optio
     if out is not None and (out.shape != (valid, h * d) or out.dtype != torch.bfloat16 or out.stride(1) != 1):
         raise ValueError(f"attention_bf16: out must be bf16 [{valid}, {h * d}] with unit column stride")
     if ATTENTION_BACKEND["name"] in (None, "fused") and 0 < valid <= l and _drop_ok(drop, valid) \
-            and takes_attention(qb, kb, vb):
+            and takes_attention(qb, kb, vb) and (out is None or not recorded(out)):
         ATTENTION_BACKEND["name"] = "fused"
         if out is not None and out.device != q.device and (valid < l or n_drop):
             raise ValueError("attention_bf16: a padded call's out must be on q's device")

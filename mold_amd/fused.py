@@ -182,6 +182,8 @@ def attention(q, k, v, valid: int, drops=None, out=None, lse=None, guard=None):
                                     scratch.data_ptr() if nbytes else None, nbytes, _stream_ptr()))
     if out is not None and res is not out:
         return out.copy_(res)
+    if out is not None:
+        torch.autograd.graph.increment_version(out)     # written in place, as a copy_ tells autograd
     return res
 
 

@@ -25,7 +25,7 @@ class _Lib:
 
     def __init__(self):
         self.calls = []
-        self.fill_lse = None     # a head's log-sum-exp
+        self.fill_lse = torch.full((H,), 50.0)     # each head's log-sum-exp
 
     def mq_attention_scratch_size(self, *a):
         return 0
@@ -34,7 +34,7 @@ class _Lib:
         batch, heads, l, valid, sb, ldo = map(int, (batch, heads, l, valid, sb, ldo))     # a trace's sizes are tensors
         self.calls.append(types.SimpleNamespace(out=out, ldo=ldo, lse=lse, guard=guard))
         assert hd == HD and ldo >= heads * HD
-        if lse and self.fill_lse is not None:
+        if lse:
             _at(lse, heads * valid, torch.float32, ctypes.c_float).view(heads, valid).copy_(
                 self.fill_lse[:, None].expand(heads, valid))
         for b in range(batch):
@@ -206,3 +206,24 @@ def test_one_row_of_out_may_have_any_stride(lib):
     one = torch.empty((1, H * HD), dtype=torch.bfloat16).as_strided((1, 1, H * HD), (3, 5, 1))
     assert torch.equal(FU.attention(q[None], k[None], v[None], 1, out=one)[0], ref)
     assert [c.ldo for c in lib.calls] == [H * HD] * 5
+
+
+@pytest.mark.parametrize("valid", [L, L - 3])
+def test_autograd_sees_out_change(lib, valid):
+    """out is written in place: a graph that saved its old values must not go on with the new ones, and an
+    out that requires gradients is recorded (or, a leaf, refused)."""
+    q, k, v = _qkv()
+    q, k, v = q, *(torch.cat([t[:, :valid], 0 * t[:, valid:]], 1) for t in (k, v))
+    out = torch.randn((valid, H * HD)).to(torch.bfloat16)
+    x = torch.ones_like(out, requires_grad=True)
+    y = (out * x).sum()
+    F.attention_bf16(q, k, v, valid=valid, out=out)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.backward()
+    leaf = torch.zeros_like(out, requires_grad=True)
+    with pytest.raises(RuntimeError):
+        F.attention_bf16(q, k, v, valid=valid, out=leaf)
+    assert not leaf.detach().any()
+    with torch.no_grad():
+        F.attention_bf16(q, k, v, valid=valid, out=leaf)
+    assert torch.equal(leaf, out)
