@@ -289,6 +289,9 @@ def text_stream(device, ctx):
     return s
 
 
+# What the last attention that PyTorch ran took ("chunked": no fused kernel serves the
+# device, so later ones do not ask again); "fused" too where only libmoldq's kernel has run,
+# which does not depend on it.
 ATTENTION_BACKEND = {"name": None}
 
 
@@ -372,9 +375,9 @@ def attention_bf16(q, k, v, valid: Optional[int] = None, guard=None, drop: Optio
     of a wider buffer), receives the result in place of a new tensor.  It may lie over
     q, k or v, and on another device where nothing is padded or masked.
 
-    Where no fused kernel serves the device, it falls back to the exact
-    head-chunked path on the valid rows (any other error propagates).  The
-    backend used is recorded in ATTENTION_BACKEND."""
+    Where PyTorch has no fused kernel for the device, its calls fall back to the exact
+    head-chunked path on the valid rows (any other error propagates;
+    ATTENTION_BACKEND)."""
     import torch
     from .fused import apart, attention, recorded, takes_attention
     h, l, d = q.shape
@@ -383,9 +386,8 @@ def attention_bf16(q, k, v, valid: Optional[int] = None, guard=None, drop: Optio
     n_drop = 0 if drop is None else max(0, drop[1] - drop[0])
     if out is not None and (out.shape != (valid, h * d) or out.dtype != torch.bfloat16 or out.stride(1) != 1):
         raise ValueError(f"attention_bf16: out must be bf16 [{valid}, {h * d}] with unit column stride")
-    if ATTENTION_BACKEND["name"] in (None, "fused") and 0 < valid <= l and _drop_ok(drop, valid) \
-            and takes_attention(qb, kb, vb) and (out is None or not recorded(out)):
-        ATTENTION_BACKEND["name"] = "fused"
+    if 0 < valid <= l and _drop_ok(drop, valid) and takes_attention(qb, kb, vb) and (out is None or not recorded(out)):
+        ATTENTION_BACKEND["name"] = ATTENTION_BACKEND["name"] or "fused"
         if out is not None and out.device != q.device and (valid < l or n_drop):
             raise ValueError("attention_bf16: a padded call's out must be on q's device")
         if guard is not None or not (valid < l or n_drop):
@@ -479,15 +481,17 @@ def attention_bf16_batch(q, k, v, valid: int, guard, drops):
     b_, h, l, d = q.shape
     per_element = lambda: torch.stack([attention_bf16(q[b], k[b], v[b], valid=valid, guard=guard, drop=drops[b])
                                        for b in range(b_)])
-    if guard is None or ATTENTION_BACKEND["name"] not in (None, "fused"):
+    if guard is None:
         return per_element()
     from .fused import attention, check_guard, takes_attention
     if 0 < valid <= l and all(_drop_ok(dr, valid) for dr in drops) and len(drops) == b_ \
             and takes_attention(q, k, v):
-        ATTENTION_BACKEND["name"] = "fused"
+        ATTENTION_BACKEND["name"] = ATTENTION_BACKEND["name"] or "fused"
         check_guard(guard, q.device)
         padded = valid < l or any(dr is not None and dr[1] > dr[0] for dr in drops)
         return attention(q, k, v, valid, drops=drops, guard=guard if padded else None)
+    if ATTENTION_BACKEND["name"] not in (None, "fused"):
+        return per_element()
     try:
         out, lse = torch.ops.aten._scaled_dot_product_efficient_attention(q, k, v, None, True)[:2]
     except RuntimeError as err:

@@ -227,3 +227,12 @@ def test_autograd_sees_out_change(lib, valid):
     with torch.no_grad():
         F.attention_bf16(q, k, v, valid=valid, out=leaf)
     assert torch.equal(leaf, out)
+
+
+def test_pytorchs_backend_does_not_decide_for_the_kernel(lib):
+    """A call of another head size that found no fused kernel leaves calls of 128 where they were."""
+    q, k, v = _qkv()
+    F.ATTENTION_BACKEND["name"] = "chunked"
+    F.attention_bf16(q, k, v)
+    F.attention_bf16_batch(q[None], k[None], v[None], L, torch.zeros(()), [None])
+    assert len(lib.calls) == 2 and F.ATTENTION_BACKEND["name"] == "chunked"
