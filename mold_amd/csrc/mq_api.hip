@@ -228,11 +228,13 @@ Plan plan_qmatmul(const mq_ctx *ctx, const mq_qtensor *w, const void *x, int x_d
     bool few = gemm_skinny_ok(w->dtype, m, n, k, tail_split);
     if (few) {
       p.tail = gemm_skinny_plan(m, n, k, ctx->cu_count, tail_split);
-      if (x_dtype == MQ_F32 && f32_in_place && aligned && ldx % 4 == 0 && gemm_skinny_reads_f32(w->dtype, n, k, p.tail))
+      // its byte offsets into x are 31 bits: f32 rows further apart are staged
+      // like any other, so that mq_qmatmul_workspace_size holds for them
+      auto reach = [&](int64_t ld) { return m * ld * 4 < (int64_t(1) << 31); };
+      if (x_dtype == MQ_F32 && f32_in_place && aligned && ldx % 4 == 0 && reach(ldx) &&
+          gemm_skinny_reads_f32(w->dtype, n, k, p.tail))
         p.stage_gemm = false;
-      // its byte offsets into x are 31 bits
-      few = m * (p.stage_gemm ? p.kp : ldx) * 4 < (int64_t(1) << 31);
-      if (!few) p.stage_gemm = p.stage_gemm || x_dtype == MQ_F32;
+      few = reach(p.stage_gemm ? p.kp : ldx);
     }
     const int64_t lda = p.stage_gemm ? p.kp : ldx;
     p.stage_bytes = p.stage_gemm ? (size_t)m * p.kp * sizeof(__bf16) : 0;

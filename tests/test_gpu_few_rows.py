@@ -109,3 +109,23 @@ def test_captured_after_reserving_the_stated_workspace(dev):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, lin.forward(x)), i
+
+
+def test_far_apart_rows_fit_the_stated_workspace(dev):
+    """f32 rows that lie too far apart for the kernel's 31-bit offsets, in a stream with exactly workspace_bytes."""
+    lin, w, b, g = _weight(dev, "Q8_0", 6144, 512, seed=6)
+    m, ldx = 64, 1 << 23
+    x = torch.empty(((m - 1) * ldx + 512,), device="cuda").as_strided((m, 512), (ldx, 1))
+    x.copy_(torch.randn((m, 512), device="cuda", generator=g))
+    y = torch.empty((m, 6144), device="cuda")
+    s = torch.cuda.Stream()
+    dev.reserve_stream_scratch(lin.matmul.workspace_bytes(m), s)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        lin.matmul.forward(x, bias=lin.bias, out=y)
+    for i in range(2):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert _err(y, x.double().cpu() @ w.t() + b) < BOUND
+        assert torch.equal(y, lin.forward(x.contiguous())), i
