@@ -520,6 +520,13 @@ __device__ __forceinline__ void put_chunk(uint8_t *tiled, int64_t plane, int nch
   *reinterpret_cast<uint4 *>(tiled + plane + ((tb * nchunks + c) * kRowTile + r) * 16) =
       make_uint4(w[0], w[1], w[2], w[3]);
 }
+// The low or high four of eight words (by value: a run-time pointer into w
+// would put it in private memory).
+__device__ __forceinline__ void put_half(uint8_t *tiled, int64_t plane, int nchunks, int64_t tb, int c, int r,
+                                         const uint32_t (&w)[8], bool high) {
+  const uint32_t v[4] = {high ? w[4] : w[0], high ? w[5] : w[1], high ? w[6] : w[2], high ? w[7] : w[3]};
+  put_chunk(tiled, plane, nchunks, tb, c, r, v);
+}
 template <typename V>
 __device__ __forceinline__ void put_record(uint8_t *tiled, int64_t plane, int size, int64_t tb, int r, int off, V v) {
   *reinterpret_cast<V *>(tiled + plane + (tb * kRowTile + r) * size + off) = v;
@@ -580,7 +587,7 @@ __device__ __forceinline__ void quantize_sub(const float (&x)[N], bool real, int
       or_lanes(hb, 4);
 #pragma unroll
       for (int i = 0; i < 8; ++i) hb[i] = real ? hb[i] : 0u;
-      if (j < 2) put_chunk(t, g.plane[2], 2, tb, j, r, j == 0 ? hb : hb + 4);
+      if (j < 2) put_half(t, g.plane[2], 2, tb, j, r, hb, j != 0);
     }
     // sub-blocks 2g and 2g + 1 are the low and high nibbles of bytes 32 g ..
 #pragma unroll
@@ -588,7 +595,7 @@ __device__ __forceinline__ void quantize_sub(const float (&x)[N], bool real, int
     or_lanes(p, 1);
 #pragma unroll
     for (int i = 0; i < 8; ++i) p[i] = real ? p[i] : 0u;
-    put_chunk(t, g.plane[FIVE ? 3 : 2], 8, tb, j, r, (j & 1) == 0 ? p : p + 4);
+    put_half(t, g.plane[FIVE ? 3 : 2], 8, tb, j, r, p, (j & 1) != 0);
     if (j == 0) {
       put_record<uint32_t>(t, g.plane[0], 4, tb, r, 0, real ? (uint32_t)dh | ((uint32_t)mh << 16) : 0u);
       put_record<uint32_t>(t, g.plane[1], 12, tb, r, 0, real ? s0 : 0u);

@@ -73,6 +73,15 @@ def test_lds_dma_kernels_leave_m0_alone_and_do_not_spill(tmp_path, src, defines,
         assert meta.get("ScratchSize", 0) == 0, (name, meta)
 
 
+def test_k_quantizers_keep_to_registers(tmp_path):
+    """Each thread's values, quants and packed words stay in registers: no private array indexed at run time."""
+    funcs = {k: v for k, v in _functions(_asm(tmp_path, "mq_quant.hip")).items()
+             if "quantize_k_kernel" in k or "lora_merge_kernel" in k}
+    assert len(funcs) == 5 * 4 + 5
+    for name, (_, meta) in funcs.items():
+        assert meta.get("ScratchSize", 0) == 0, (name, meta)
+
+
 VMEM_LOAD = re.compile(r"^\s*(global_|buffer_|flat_)load")
 
 
