@@ -188,13 +188,35 @@ def _targets(patches: List[LoraPatch], base_rows: int):
         yield p, off, size
 
 
+# Mean rank over a weight's rows up to which one pass is the faster.  It reads a patch's
+# factors again for every 16 or 32 rows, mq_lora_apply for every 64: per rank and value of
+# a [21504, 3072] weight 1.3 times the time, against the passes over the f32 weight that
+# it saves (Q3_K's cheap search leaves the fewest).  One pass / separate calls, us, one patch
+# of that weight at rank 32, 128, 256 and 512: Q6_K 456 / 582, 743 / 763, 1180 / 1017,
+# 2958 / 1574; Q5_K at 128, 192 and 256: 0.87, 0.95 and 1.04 of them.
+_ONE_PASS_RANK = {GgmlDType.Q2_K: 160, GgmlDType.Q3_K: 96, GgmlDType.Q4_K: 240, GgmlDType.Q5_K: 208, GgmlDType.Q6_K: 144}
+# What a further separate call costs, in the same unit of ranks times values (four patches
+# of rank 256 on [768, 768]: one pass 0.44 - 0.54 of the separate calls, on [3072, 3072]
+# 0.85 - 0.95, on [3072, 12288] 0.96 - 1.20).
+_ONE_PASS_CALL = 1 << 30
+
+
+def _one_pass(dtype: GgmlDType, n: int, k: int, ranks_rows) -> bool:
+    """Whether mq_lora_merge takes these patches ((rank, rows) each) in less time."""
+    limit = _ONE_PASS_RANK.get(dtype)
+    if limit is None or not 1 <= len(ranks_rows) <= _lib.MQ_LORA_MAX_PATCHES:
+        return False
+    return k * sum(r * rows for r, rows in ranks_rows) <= limit * n * k + (len(ranks_rows) - 1) * _ONE_PASS_CALL
+
+
 def patch_qtensor(qt: QTensor, patches: List[LoraPatch]) -> Tuple[QTensor, int]:
     """One targeted tensor (lora.rs:748-849) on the device: dequantize to f32,
     apply each patch, re-quantize to the original type; a k-quant in one pass
-    (mq_lora_merge: the same blocks).  Returns (new tensor, patches applied)."""
+    up to the ranks where that is faster (mq_lora_merge: the same blocks).
+    Returns (new tensor, patches applied)."""
     n, k = qt.shape
     todo = list(_targets(patches, n))
-    if qt.dtype().block_size() == 256 and 1 <= len(todo) <= _lib.MQ_LORA_MAX_PATCHES \
+    if _one_pass(qt.dtype(), n, k, [(p.a.shape[0], size) for p, _, size in todo]) \
             and all(off >= 0 and size >= 0 and p.a.shape[0] >= 1 for p, off, size in todo):
         keep = [_device_factors(p.b, p.a, f"cuda:{qt.device.ordinal}", size, k) for p, _, size in todo]
         arr = (_lib.LoraPatchC * len(todo))(*[

@@ -66,6 +66,22 @@ def test_patch_qtensor_takes_it_and_falls_back(dev):
         assert applied == count and np.array_equal(out.data(), _chain(qt, [(0, b, a, 0.5) for b, a in fs])), (t, count)
 
 
+@pytest.mark.parametrize("t,rank,one", [("Q4_K", 32, True), ("Q4_K", 240, True), ("Q4_K", 241, False), ("Q3_K", 97, False),
+                                         ("Q6_K", 512, False), ("Q2_K", 160, True), ("Q5_K", 300, False)])
+def test_high_ranks_take_the_separate_calls(dev, t, rank, one, monkeypatch):
+    """Where they are faster; the blocks are the same."""
+    g = torch.Generator(device="cuda").manual_seed(rank)
+    rn = lambda *s: torch.randn(s, device="cuda", generator=g)
+    qt = QTensor.quantize(dev, rn(131, 512) * 0.02, GgmlDType[t])
+    b, a = rn(131, rank) * 0.02, rn(rank, 512) * 0.05
+    merges, lib = [], _lib.load()
+    real = lib.mq_lora_merge
+    monkeypatch.setattr(lib, "mq_lora_merge", lambda *args: merges.append(1) or real(*args))
+    out, _ = L.patch_qtensor(qt, [L.LoraPatch(a, b, 0.5, L.LoraTarget("w"))])
+    assert len(merges) == one
+    assert np.array_equal(out.data(), _chain(qt, [(0, b, a, 0.5)])) and np.array_equal(out.data(), _merge(qt, [(0, b, a, 0.5)]))
+
+
 def test_refuses(dev):
     g = torch.Generator(device="cuda").manual_seed(1)
     rn = lambda *s: torch.randn(s, device="cuda", generator=g)

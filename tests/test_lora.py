@@ -118,3 +118,17 @@ def test_adapter_alpha_only_from_rank0_f32(tmp_path):
     assert effs["single_blocks.0.linear2.weight"] == 0.5 * 8.0 / 4     # scale * alpha / rank
     for i in (1, 2, 3):
         assert effs[f"single_blocks.{i}.linear2.weight"] == 0.5       # alpha dropped
+
+
+def test_one_pass_up_to_the_rank_where_it_is_faster():
+    """Mean rank over the weight's rows; further patches each save a call; 32-element types never."""
+    from mold_amd import GgmlDType, _lib
+    from mold_amd.lora import _one_pass
+    n, k = 21504, 3072
+    for t, limit in (("Q2_K", 160), ("Q3_K", 96), ("Q4_K", 240), ("Q5_K", 208), ("Q6_K", 144)):
+        assert _one_pass(GgmlDType[t], n, k, [(limit, n)]) and not _one_pass(GgmlDType[t], n, k, [(limit + 1, n)])
+        assert _one_pass(GgmlDType[t], n, k, [(4 * limit, n // 4)])            # a quarter of the rows
+        assert not _one_pass(GgmlDType[t], n, k, [(2 * limit, n // 2), (2 * limit, n // 2), (limit, n)])
+    assert _one_pass(GgmlDType.Q4_K, 768, 768, [(256, 192)] * 4)
+    assert not _one_pass(GgmlDType.Q8_0, 96, 256, [(4, 96)]) and not _one_pass(GgmlDType.Q4_K, n, k, [])
+    assert not _one_pass(GgmlDType.Q4_K, n, k, [(1, n)] * (_lib.MQ_LORA_MAX_PATCHES + 1))
