@@ -186,6 +186,19 @@ def test_other_calls_keep_pytorch_attention():
     assert not FU.takes_attention(*small) and attention_bf16(*small).shape == (64, 128)
 
 
+@gpu
+@pytest.mark.parametrize("name,args", [
+    ("test_padded_attention_matches_reference", (295, 512)), ("test_padded_attention_matches_reference", (1000, 1024)),
+    ("test_padded_attention_matches_reference", (512, 512)), ("test_batched_padded_attention_with_dropped_keys", ()),
+    ("test_padded_attention_ill_conditioned_rows_recomputed", ()), ("test_padded_attention_guard_and_step_rerun", ())])
+def test_pytorch_route_of_padded_calls(name, args, monkeypatch):
+    """The zero-key correction, the recompute and the masked keys of calls the kernel does not take."""
+    from tests import test_gpu_glue
+    monkeypatch.setattr(FU, "takes_attention", lambda q, k, v: False)
+    monkeypatch.setattr(FU, "attention", None)
+    getattr(test_gpu_glue, name)(*args)
+
+
 def test_argument_checks():
     from mold_amd import _lib
     lib = _lib.load()
