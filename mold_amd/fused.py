@@ -114,6 +114,14 @@ def recorded(*inputs) -> bool:
             or torch.jit.is_tracing() or (torch._C._is_torch_function_mode_enabled() and _recording_mode()))
 
 
+def takes_shape(shape) -> bool:
+    """mq_attention_bf16's sizes: heads of 128, up to 2^23 rows and 2^20 heads over the batch."""
+    if len(shape) not in (3, 4) or shape[-1] != HEAD_DIM:
+        return False
+    heads = shape[-3] * (shape[0] if len(shape) == 4 else 1)
+    return 0 < heads <= 1 << 20 and 0 < shape[-2] <= 1 << 23
+
+
 def takes_attention(q, k, v) -> bool:
     """Whether `attention` computes these q, k, v: bf16 [.., H, L, 128] of one shape on one
     GPU, contiguous and 16-byte aligned, with nothing recording the call."""
@@ -122,8 +130,7 @@ def takes_attention(q, k, v) -> bool:
         if type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda or t.dtype != torch.bfloat16 \
                 or t.shape != q.shape or t.device != q.device or not t.is_contiguous() or t.data_ptr() % 16:
             return False
-    return (q.dim() in (3, 4) and q.shape[-1] == HEAD_DIM and 0 < q.numel() and q.shape[-2] <= 1 << 23
-            and not recorded(q, k, v))
+    return takes_shape(q.shape) and not recorded(q, k, v)
 
 
 def apart(out, *inputs) -> bool:

@@ -236,3 +236,11 @@ def test_pytorchs_backend_does_not_decide_for_the_kernel(lib):
     F.attention_bf16(q, k, v)
     F.attention_bf16_batch(q[None], k[None], v[None], L, torch.zeros(()), [None])
     assert len(lib.calls) == 2 and F.ATTENTION_BACKEND["name"] == "chunked"
+
+
+def test_sizes_the_entry_refuses_stay_with_pytorch():
+    assert FU.takes_shape((24, 4608, 128)) and FU.takes_shape((2, 24, 4608, 128)) and FU.takes_shape((1 << 20, 1, 128))
+    assert FU.takes_shape((2, 1 << 19, 1, 128)) and FU.takes_shape((1, 1 << 23, 128))
+    for shape in ((1 + (1 << 20), 1, 128), (2, 1 + (1 << 19), 1, 128), (1, 1 + (1 << 23), 128), (0, 4, 128), (4, 0, 128),
+                  (0, 4, 4, 128), (4, 4, 64), (4, 128), (1, 1, 4, 4, 128)):
+        assert not FU.takes_shape(shape), shape
