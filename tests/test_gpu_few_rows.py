@@ -86,6 +86,38 @@ def test_epilogues_strides_and_unsplit(dev, m):
     assert _err(whole, ref) < BOUND
 
 
+@pytest.mark.parametrize("k", [256, 3072])
+def test_whole_and_ragged_blocks_of_rows(dev, k):
+    """Whole 32-row blocks and the last one, columns with and without GELU in one wave, the residual's rows, in one part of K."""
+    lin, w, b, g = _weight(dev, "Q4_K", 333, k, seed=7)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    dev.set_stream_tail_split(s, False)
+    gate = torch.randn(333, device="cuda", generator=g)
+    with torch.cuda.stream(s):
+        for m in (1, 3, 8, 9, 31, 32, 33, 60, 63, 64):
+            x = torch.randn((m, k), device="cuda", generator=g).bfloat16()
+            ref = x.double().cpu() @ w.t() + b
+            gelu = ref.clone()
+            gelu[:, 77:] = torch.nn.functional.gelu(ref[:, 77:], approximate="tanh")
+            buf = torch.full((m + 2, 400), 5.0, device="cuda")
+            res, full = buf[1:m + 1, 30:363], torch.full((m + 2, 333), 3.0, device="cuda")
+            r0 = torch.randn((m, 333), device="cuda", generator=g)
+            res.copy_(r0)
+            lin.gated_add(x, gate, res)
+            s.synchronize()
+            assert _err(res, r0.double().cpu() + gate.double().cpu() * ref) < BOUND, m
+            res.fill_(5.0)
+            assert bool((buf == 5.0).all()), m
+            if m > 8:                                           # up to 8 rows are the GEMV's
+                for dt in (torch.float32, torch.bfloat16):
+                    out = full.to(dt)
+                    lin.matmul.forward(x, bias=lin.bias, act=ACT_GELU_TANH, act_from=77, out=out[1:m + 1])
+                    s.synchronize()
+                    assert _err(out[1:m + 1], gelu) < BOUND and bool((out[0] == 3).all()) and bool((out[m + 1] == 3).all()), m
+    dev.set_stream_tail_split(s, True)
+
+
 def test_y_over_f32_x(dev):
     """y written over f32 x: x is read whole before any of y is written."""
     lin, w, b, g = _weight(dev, "Q8_0", 512, 512, seed=4)
