@@ -681,7 +681,7 @@ __global__ __launch_bounds__(512, 2) void gemm_skinny_kernel(
   OUT *yc = y + 4 * h * ldy + col;
   // Activation chosen once, rows checked in the last block only.  Checked per
   // element, with the GELU's code between the stores, the epilogue alone cost 5
-  // us at 64 rows (64 x 256 -> 1024 Q4_K 9.9 us, now 5.2; 33 rows 7.6, now 5.5).
+  // us at 64 rows (64 x 256 -> 1024 Q4_K 9.9 us, now 5.4; 33 rows 7.6, now 5.4).
   auto emit = [&]<bool kGelu>() {
     float g = 0.f;
     if constexpr (GATED) g = gate[col];
@@ -1005,8 +1005,22 @@ int gemm_tile_m(int type, int64_t m, int64_t n, int64_t k, int cus) {
 // that (us, before / now, bf16 x): 9 x 4096 -> 4096 Q8_0 16.2 / 10.9, 64
 // 16.3 / 14.5, 77 17.3 / 15.7, 77 x 4096 -> 10240 28.5 / 21.8, 32 x 12288 ->
 // 3072 Q2_K 19.1 / 13.2, 77 x 3072 -> 3072 Q4_K 15.6 / 12.2.
+// Its parts of K are chunks of 512 or 256 columns, the tiles' are units of 128
+// (Q8_0) or 256, so on a small weight a short K leaves it fewer parts, and the
+// tiles are faster (bf16 x): 64 x 1024 -> 1024 Q8_0 6.9 us against 8.1 here, Q4_0
+// 6.9 / 8.0, 64 x 2048 -> 1024 7.6 / 8.4, 96 x 512 -> 1024 Q8_0 6.5 / 7.5; past the
+// lines 64 x 2560 -> 1024 Q4_0 8.6 / 8.5, 64 x 2048 -> 4096 11.3 / 10.1.  f32 x
+// takes the same kernel as its bf16 rounding, so that both give the same y: it is
+// staged for the tiles and would be up to 10 % faster here; where it gains more
+// than bf16 loses, the few rows stay here (32 x 768 -> 512 Q8_0 6.0 / 7.0 bf16, 8.8
+// / 7.4 f32; 64 x 256 -> 1024 Q4_K 4.8 / 5.4, 7.6 / 5.7).  Wide weights leave it long
+// parts: 64 x 8192 -> 12288 Q8_0 29.2 / 32.9, 3072 -> 12288 17.3 / 18.4.
 bool gemm_skinny_ok(int type, int64_t m, int64_t n, int64_t k, bool split) {
-  return m <= 96 && (m <= 64 || split) && (m <= 32 || n <= 112 * 128) && k % gemm_unit_k(type) == 0;
+  if (m > 96 || (m > 64 && !split) || (m > 32 && n > 112 * 128) || k % gemm_unit_k(type) != 0) return false;
+  if (m <= 32 || !split) return true;
+  const bool fine = gemm_unit_k(type) == 128;  // the tiles' finer units
+  if (m > 64) return !(n <= 2048 && k >= 512 && k <= (fine ? 3072 : 2048));
+  return !(n <= 2048 && k > 512 && k <= 2048) && !(n >= 10240 && k >= (fine ? 2560 : 6144));
 }
 
 // Its plan: a 128-feature tile holds a CU's LDS alone (two fit up to 32 rows),
