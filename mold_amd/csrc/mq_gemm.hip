@@ -1064,7 +1064,9 @@ GemmTail gemm_tail_plan(int type, int64_t m, int64_t n, int64_t k, int cus, bool
     // Less than one round of 256-row tiles: 128-row tiles, split by their own
     // rule, where they are estimated clearly cheaper: fewer padded rows (300 x
     // 3072 -> 9216 Q4_K 41.8 -> 35.7 us, 300 x 5120 -> 5120 Q6_K 41.4 -> 34.4) or
-    // no partial sums at a good fill (512 x 3072 -> 12288 52.7 -> 48.3).
+    // no partial sums at a good fill (512 x 3072 -> 12288 52.7 -> 48.3).  Not on a
+    // stream that does not split K: beside the other stream's GEMMs they gain
+    // nothing (a FLUX forward of six blocks 8.46 ms with them, 8.43 without).
     const int64_t t256 = ((m + 255) / 256) * ((n + 255) / 256), t128 = ((m + 127) / 128) * ((n + 127) / 128);
     if (t256 < cus) {
       int64_t rem = 0;

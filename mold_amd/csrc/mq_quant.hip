@@ -463,10 +463,9 @@ __global__ __launch_bounds__(64) void quantize_tiled_kernel(const void *__restri
 // stored by one lane straight into the device layout (rows past n as zeros).
 // With one thread a super-block (the values, quants and search candidates in
 // private memory, raw blocks to a staging buffer, then a repack pass) Q4_K
-// [21504, 3072] took 1022 + 39 us, now 640 (VALU-bound: about 430 operations a
-// value at one per lane and cycle); [8192, 3072] whole calls, before -> now:
-// Q2_K 496 -> 242 us, Q3_K 428 -> 133, Q4_K 567 -> 298, Q5_K 538 -> 247, Q6_K
-// 383 -> 182.
+// [21504, 3072] took 1022 + 39 us, now 640 (VALU-bound: 438 instructions a value,
+// a wave instruction every 3.1 cycles per SIMD at 2.1 GHz); [8192, 3072] whole calls, before -> now: Q2_K 496 ->
+// 242 us, Q3_K 428 -> 133, Q4_K 567 -> 298, Q5_K 538 -> 247, Q6_K 383 -> 182.
 
 // v combined over the W lanes of a super-block by or / by maximum (values never NaN there).
 template <int W>
@@ -774,13 +773,14 @@ __global__ __launch_bounds__(256) void quantize_k_kernel(const void *__restrict_
 // does), plus each patch's (b . a) * scale on its rows, quantized again; the
 // steps and their order are those of dequantize, lora_apply per patch and
 // quantize, so the blocks are the same.  Bound by the search's VALU work as
-// quantize_k_kernel is: the rank's fmas add 32 operations a value at rank 32 to
-// about 430, where the three passes moved 28 bytes a value through HBM (Q4_K
-// [21504, 3072], four rank-32 patches: 55 + 234 + 640 us, in one pass 700; the
-// merge call 1003 -> 728).  A patch's a
-// (kLoraR ranks of the workgroup's 256 columns) and b are staged in LDS, a
-// with the lanes' 16-byte pieces side by side (piece c of sub-block j at
-// c * lanes + j: the lanes of a row read 128 or 256 consecutive bytes).
+// quantize_k_kernel is: decode and rank-32 patches add 52 instructions a value to
+// 438, where the separate passes moved 17 bytes a value through HBM (written 4,
+// read and written 4 + 4 by the patches, read 4, the blocks 0.6 each way; Q4_K
+// [21504, 3072], four rank-32 patches: 55 + 234 + 640 us, in one pass 685; the
+// merge call 1003 -> 721).  A patch's a (kLoraR ranks of the workgroup's 256
+// columns) and b are staged in LDS, a with the lanes' 16-byte pieces side by side
+// (piece c of sub-block j at c * lanes + j: the lanes of a row read 128 or 256
+// consecutive bytes).
 constexpr int kLoraR = 32;
 
 template <int TYPE>

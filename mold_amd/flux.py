@@ -360,7 +360,8 @@ def attention_bf16(q, k, v, valid: Optional[int] = None, guard=None, drop: Optio
     PyTorch's kernels do: each of the n_pad zero keys adds exp(0) = 1 to a row's
     softmax denominator, so out = out_pad / s with s = 1 - n_pad exp(-lse), the
     row's share of mass on its valid keys, which loses precision once s falls
-    under PAD_MIN_SHARE (every valid score below about -10).  On either path such
+    under PAD_MIN_SHARE (every valid score below about -10).  On either path (the
+    kernel's rows need none of it: a call's decisions are the same on both) such
     rows are reported or recomputed in f32 over the valid keys: with `guard` None
     this call finds them (one host synchronization) and recomputes their heads;
     with `guard`, a 0-dim f32 device tensor, it only raises guard to the largest
