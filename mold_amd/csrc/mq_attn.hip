@@ -493,7 +493,7 @@ extern "C" int mq_attention_bf16(const void *q, const void *k, const void *v, in
   if (head_dim != kHd) return invalid("mq_attention_bf16: head_dim must be 128");
   if (batch < 0 || heads <= 0 || valid < 0 || valid > l_total)
     return invalid("mq_attention_bf16: negative batch, heads < 1, or valid outside 0 .. l_total");
-  if (l_total > (int64_t(1) << 23) || batch * heads > (int64_t(1) << 20))
+  if (l_total > (int64_t(1) << 23) || batch > (int64_t(1) << 20) / heads)
     return invalid("mq_attention_bf16: l_total above 2^23 or more than 2^20 heads");
   if (!q || !k || !v || !out) return invalid("mq_attention_bf16: NULL pointer");
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out) || !aligned16(scratch) || ldo % 8 ||

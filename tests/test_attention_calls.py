@@ -244,3 +244,12 @@ def test_sizes_the_entry_refuses_stay_with_pytorch():
     for shape in ((1 + (1 << 20), 1, 128), (2, 1 + (1 << 19), 1, 128), (1, 1 + (1 << 23), 128), (0, 4, 128), (4, 0, 128),
                   (0, 4, 4, 128), (4, 4, 64), (4, 128), (1, 1, 4, 4, 128)):
         assert not FU.takes_shape(shape), shape
+
+
+@pytest.mark.parametrize("batch,heads", [(1 << 62, 4), (1 << 21, 1), (1, (1 << 20) + 1), ((1 << 20) // 3 + 1, 3)])
+def test_c_entry_refuses_more_heads_than_it_counts(batch, heads):
+    """Also where batch * heads does not fit 64 bits (addresses only: refused before any launch)."""
+    from mold_amd import _lib
+    rc = _lib.load().mq_attention_bf16(4096, 4096, 4096, batch, heads, 64, HD, 64, None, 1 << 40, 0, heads * HD, None, None, None, 0,
+                                       None)
+    assert rc == -1 and b"2^20 heads" in _lib.load().mq_last_error()
