@@ -107,18 +107,22 @@ def recorded(*inputs) -> bool:
     forward-mode AD, a dispatch or function mode, a compiler, a trace): it needs operations
     PyTorch knows."""
     import torch
-    return ((torch.is_grad_enabled() and any(t.requires_grad for t in inputs))
-            or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch.autograd.forward_ad._current_level >= 0
-            or torch._C._len_torch_dispatch_stack() != 0 or torch.compiler.is_compiling()
-            or torch.jit.is_tracing() or (torch._C._is_torch_function_mode_enabled() and _recording_mode()))
+    if torch.is_grad_enabled():
+        for t in inputs:
+            if t.requires_grad:
+                return True
+    c = torch._C
+    return (c._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0
+            or c._len_torch_dispatch_stack() != 0 or torch.compiler.is_compiling() or c._is_tracing()
+            or (c._is_torch_function_mode_enabled() and _recording_mode()))
 
 
 def takes_shape(shape) -> bool:
     """mq_attention_bf16's sizes: heads of 128, up to 2^23 rows and 2^20 heads over the batch."""
-    if len(shape) not in (3, 4) or shape[-1] != HEAD_DIM:
+    n = len(shape)
+    if n not in (3, 4) or shape[-1] != HEAD_DIM:
         return False
-    heads = shape[-3] * (shape[0] if len(shape) == 4 else 1)
+    heads = shape[0] if n == 3 else shape[0] * shape[1]
     return 0 < heads <= 1 << 20 and 0 < shape[-2] <= 1 << 23
 
 
@@ -126,26 +130,31 @@ def takes_attention(q, k, v) -> bool:
     """Whether `attention` computes these q, k, v: bf16 [.., H, L, 128] of one shape on one
     GPU, contiguous and 16-byte aligned, with nothing recording the call."""
     import torch
+    shape, device = q.shape, q.device
     for t in (q, k, v):
-        if type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda or t.dtype != torch.bfloat16 \
-                or t.shape != q.shape or t.device != q.device or not t.is_contiguous() or t.data_ptr() % 16:
+        if type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda or t.dtype is not torch.bfloat16 \
+                or t.shape != shape or t.device != device or not t.is_contiguous() or t.data_ptr() % 16:
             return False
-    return takes_shape(q.shape) and not recorded(q, k, v)
+    return takes_shape(shape) and not recorded(q, k, v)
 
 
 def apart(out, *inputs) -> bool:
     """Whether out's bytes, first to last, lie clear of the (contiguous) inputs'."""
-    size = out.element_size()
-    lo = out.data_ptr()
-    hi = lo + size * (1 + sum((n - 1) * st for n, st in zip(out.shape, out.stride())))
-    return all(t.device != out.device or hi <= t.data_ptr() or t.data_ptr() + t.numel() * t.element_size() <= lo
-               for t in inputs)
+    lo, last = out.data_ptr(), 0
+    for n, stride in zip(out.shape, out.stride()):
+        last += (n - 1) * stride
+    hi = lo + (last + 1) * out.element_size()
+    for t in inputs:
+        at = t.data_ptr()
+        if at < hi and lo < at + t.nbytes and t.device == out.device:
+            return False
+    return True
 
 
 def check_guard(guard, device):
     """The kernels raise a guard with a 4-byte atomic at its address."""
     import torch
-    if guard.dtype != torch.float32 or guard.numel() != 1 or guard.device != device:
+    if guard.dtype is not torch.float32 or guard.numel() != 1 or guard.device != device:
         raise ValueError("attention: guard must be a one-element f32 tensor on q's device")
 
 
