@@ -1012,8 +1012,8 @@ int gemm_tile_m(int type, int64_t m, int64_t n, int64_t k, int cus) {
 // lines 64 x 2560 -> 1024 Q4_0 8.6 / 8.5, 64 x 2048 -> 4096 11.3 / 10.1.  f32 x
 // takes the same kernel as its bf16 rounding, so that both give the same y: it is
 // staged for the tiles and would be up to 10 % faster here; where it gains more
-// than bf16 loses, the few rows stay here (32 x 768 -> 512 Q8_0 6.0 / 7.0 bf16, 8.8
-// / 7.4 f32; 64 x 256 -> 1024 Q4_K 4.8 / 5.4, 7.6 / 5.7).  Wide weights leave it long
+// than bf16 loses, the few rows stay here (32 x 768 -> 512 Q8_0 6.1 / 7.0 bf16, 8.2
+// / 7.5 f32; 64 x 256 -> 1024 Q4_K 4.8 / 5.3, 6.9 / 6.1).  Wide weights leave it long
 // parts: 64 x 8192 -> 12288 Q8_0 29.2 / 32.9, 3072 -> 12288 17.3 / 18.4.
 bool gemm_skinny_ok(int type, int64_t m, int64_t n, int64_t k, bool split) {
   if (m > 96 || (m > 64 && !split) || (m > 32 && n > 112 * 128) || k % gemm_unit_k(type) != 0) return false;

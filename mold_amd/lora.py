@@ -189,9 +189,8 @@ def _targets(patches: List[LoraPatch], base_rows: int):
 
 
 # Mean rank over a weight's rows up to which one pass is the faster.  It reads a patch's
-# factors again for every 16 or 32 rows, mq_lora_apply for every 64: per rank and value of
-# a [21504, 3072] weight 1.3 times the time, against the passes over the f32 weight that
-# it saves (Q3_K's cheap search leaves the fewest).  One pass / separate calls, us, one patch
+# factors again for every 16 or 32 rows, mq_lora_apply for every 64: 3.2 us a rank against
+# 1.9 on a Q6_K [21504, 3072], beside the passes over the f32 weight that it saves.  One pass / separate calls, us, one patch
 # of that weight at rank 32, 128, 256 and 512: Q6_K 456 / 582, 743 / 763, 1180 / 1017,
 # 2958 / 1574; Q5_K at 128, 192 and 256: 0.87, 0.95 and 1.04 of them.
 _ONE_PASS_RANK = {GgmlDType.Q2_K: 160, GgmlDType.Q3_K: 96, GgmlDType.Q4_K: 240, GgmlDType.Q5_K: 208, GgmlDType.Q6_K: 144}
